@@ -1,13 +1,13 @@
 // Top-k block selection for gfx950: block scorer and per-(sequence, kv head)
 // radix select fused in one launch, one 1024-thread workgroup per (sequence,
-// kv head).  A whole score row stays inside one workgroup, so the launch needs
+// kv head) (rows of more than 1024 blocks: two launches, below).  A whole score row stays inside one workgroup, so the launch needs
 // no cross-workgroup synchronisation (an agent-scope fence writes back the
 // XCD's L2 and costs far more than the work here).
 //
 //   scoring: score_j = (mean_g q_g) . k_bar_j / sqrt(D); one k_bar row per 16
 //   lanes (4 rows per wave-wide load), 16 (bf16) or 8 (fp32) rows per lane in
 //   flight, DPP row sums;
-//   scores land in LDS (and in global memory when requested or too many).
+//   scores land in LDS (and in global memory when requested).
 //   selection:
 //     * forced blocks: the first forced_first and last forced_last valid blocks;
 //     * the k_eff largest remaining scores by an MSB-first 8-bit radix select
@@ -18,6 +18,8 @@
 //       block ids in ascending order.
 //   The rule is the group-mean score + torch.topk of CBG/methods/quest.py:91-103
 //   with the mean key (k_bar) as the block representative.
+#include <type_traits>
+
 #include "plan.hpp"
 #include "topk_select.hpp"
 
@@ -28,6 +30,7 @@ namespace {
 constexpr int kSelThreads = 1024;
 constexpr int kSelWaves = kSelThreads / 64;
 constexpr int kMaxLdsScores = 8192;
+constexpr int kOneLaunchBlocks = 1024;  // rows scored and selected by one workgroup in one launch
 
 struct SelectParams {
   const void* q;
@@ -45,13 +48,12 @@ struct SelectParams {
   float* scores;  // [batch*Hkv, nb_max] or null
   int32_t n_kv_heads;
   float score_scale;   // 1 / (G * sqrt(D)) (mean key) or 1 / G (Quest)
-  int32_t lds_scores;  // score rows of up to this many blocks stay in LDS
 };
 
 template <int D, int G, bool QF32, bool KBF16, bool QUEST>
 __global__ __launch_bounds__(kSelThreads) void ia_condition_block_select_topk(SelectParams p) {
   constexpr int DPL = D / 16;
-  extern __shared__ float sc_lds[];  // p.lds_scores floats
+  extern __shared__ float sc_lds[];  // p.nb_max floats
   __shared__ TopkLds<kSelThreads> sel_lds;
 
   const int lane = threadIdx.x & 63;
@@ -63,7 +65,6 @@ __global__ __launch_bounds__(kSelThreads) void ia_condition_block_select_topk(Se
   const int bh = b * p.n_kv_heads + h;
   const int seq_len = max(p.seq_lens[b], 0);
   const int nb = min((seq_len + p.block_size - 1) / p.block_size, p.nb_max);
-  const bool in_lds = nb <= p.lds_scores;
   float* sc_row = p.scores ? p.scores + (int64_t)bh * p.nb_max : nullptr;
 
   // ---- q rows (loaded first, summed after the first k_bar loads are in flight)
@@ -164,7 +165,7 @@ __global__ __launch_bounds__(kSelThreads) void ia_condition_block_select_topk(Se
         const int j = base + kRowsPerStep * t + 4 * wave + r;
         if (c16 % kCopies == 0 && base + kRowsPerStep * t < nb && j < nb) {
           const float a = v[k] * p.score_scale;
-          if (in_lds) sc_lds[j] = a;
+          sc_lds[j] = a;
           if (sc_row) sc_row[j] = a;
         }
       }
@@ -182,7 +183,7 @@ __global__ __launch_bounds__(kSelThreads) void ia_condition_block_select_topk(Se
                               : block_score<DPL, KBF16>(w1, qm, p.score_scale);
         const int j = base + kRowsPerStep * t + 4 * wave + r;
         if (c16 == 0 && j < nb) {
-          if (in_lds) sc_lds[j] = a;
+          sc_lds[j] = a;
           if (sc_row) sc_row[j] = a;
         }
       }
@@ -193,7 +194,7 @@ __global__ __launch_bounds__(kSelThreads) void ia_condition_block_select_topk(Se
     for (int j = nb + threadIdx.x; j < p.nb_max; j += kSelThreads) sc_row[j] = kNegInf;
   }
   __syncthreads();
-  auto key_at = [&](int j) -> u32 { return order_key(in_lds ? sc_lds[j] : sc_row[j]); };
+  auto key_at = [&](int j) -> u32 { return order_key(sc_lds[j]); };
 
   // ---- selection (forced blocks, radix-select threshold, ordered compaction)
   const int k_b = p.k_per_seq ? max(p.k_per_seq[b], 0) : p.k;
@@ -203,6 +204,202 @@ __global__ __launch_bounds__(kSelThreads) void ia_condition_block_select_topk(Se
   if (threadIdx.x == 0) p.n_sel[bh] = n;
 }
 
+// ---------------------------------------------------------------- long rows: two launches
+//
+// A row of many blocks keeps one workgroup of the kernel above streaming its keys alone
+// (one CU, ~40 GB/s: 99 us for 8 rows of 15,626 bf16 D = 128 blocks, 248 CUs idle).  Long
+// rows are therefore scored by a launch over the whole device, and a second launch of one
+// workgroup per row selects from the stored scores (the same score arithmetic and rule,
+// so the same bits).  Those 8 rows then take 9 + 11 us: the scorer reads 32 MB at 3.5 TB/s
+// (a workgroup lives for one round trip), and the selection is bound by one CU's vector
+// instructions, about 80 per key over its passes.  Scores held by the threads in registers,
+// strided so that the row is read coalesced: 20.8 us for both launches against 24.1 with
+// the row staged in LDS and 24.7 with 16 consecutive scores per thread (their loads touch
+// 64 lines per instruction).
+
+// Block scores [row, nb_max] (-inf past a row's end): 256 threads score kBlocks
+// consecutive blocks of one row (128 of bf16 D = 128 keys; twice as many per workgroup
+// measured 0.2-1.5 us slower); every key row of a lane is requested before any is used.
+template <int D, bool KBF16, bool QUEST>
+struct ScoreShape {
+  static constexpr int kRowWords = D / 16 * (KBF16 ? 2 : 4) / 4;             // words per lane per key row
+  static constexpr int kSteps = 32 / kRowWords / (QUEST ? 2 : 1);            // key rows (pairs) per lane in flight
+  static constexpr int kBlocks = 16 * kSteps;                                // blocks per workgroup
+};
+
+template <int D, bool KBF16, bool QUEST>
+__global__ __launch_bounds__(256) void ia_condition_block_scores(SelectParams p, int group, int q_f32, int q_vec) {
+  using S = ScoreShape<D, KBF16, QUEST>;
+  constexpr int DPL = D / 16;
+  constexpr int EB = KBF16 ? 2 : 4;
+  constexpr int NWR = S::kRowWords;
+  constexpr int NS = S::kSteps;
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int c16 = lane & 15;
+  const int r = lane >> 4;
+  const int h = blockIdx.y;
+  const int b = blockIdx.z;
+  const int base = blockIdx.x * S::kBlocks;
+  const int seq_len = max(p.seq_lens[b], 0);
+  const int nb = min((seq_len + p.block_size - 1) / p.block_size, p.nb_max);
+  float* sc_row = p.scores + ((int64_t)b * p.n_kv_heads + h) * p.nb_max;
+  if (base >= nb) {
+    for (int j = base + threadIdx.x; j < min(base + S::kBlocks, p.nb_max); j += 256) sc_row[j] = kNegInf;
+    return;
+  }
+  // keys: in step t, wave w handles row base + 16 t + 4 w + r (rows past nb re-read row nb - 1)
+  const int64_t head = ((int64_t)b * p.kb_batch_stride + (int64_t)h * p.kb_head_stride) * EB;
+  const char* kb = reinterpret_cast<const char*>(p.k_bar) + head;
+  const char* kn = reinterpret_cast<const char*>(QUEST ? p.k_min : p.k_bar) + head;
+  u32 w1[NS][NWR], w2[QUEST ? NS : 1][NWR];
+  auto load_row = [&](const char* rowp, u32* w) {
+    if constexpr (NWR >= 4) {
+#pragma unroll
+      for (int v4 = 0; v4 < NWR; v4 += 4) {
+        const u32x4_t x = ld_stream16(rowp + 4 * v4);
+        w[v4] = x[0]; w[v4 + 1] = x[1]; w[v4 + 2] = x[2]; w[v4 + 3] = x[3];
+      }
+    } else {
+      const u32x2_t x = ld_stream8(rowp);
+      w[0] = x[0]; w[1] = x[1];
+    }
+  };
+#pragma unroll
+  for (int t = 0; t < NS; ++t) {
+    const int64_t off = ((int64_t)min(base + 16 * t + 4 * wave + r, nb - 1) * D + c16 * DPL) * EB;
+    load_row(kb + off, w1[t]);
+    if constexpr (QUEST) load_row(kn + off, w2[t]);
+  }
+  // mean key: qm = sum_g q_g; Quest: qm = sum_g q_g+, qn = sum_g q_g- (g ascending)
+  float qm[DPL], qn[DPL];
+#pragma unroll
+  for (int e = 0; e < DPL; ++e) {
+    qm[e] = 0.f;
+    qn[e] = 0.f;
+  }
+  for (int g = 0; g < group; ++g) {
+    const int64_t row = (int64_t)b * p.q_batch_stride + (int64_t)(h * group + g) * p.q_row_stride + c16 * DPL;
+    float x[DPL];
+    if (q_f32) {
+      const float* q0 = reinterpret_cast<const float*>(p.q) + row;
+      if (q_vec) {
+#pragma unroll
+        for (int e = 0; e < DPL; e += 4) {
+          const f32x4_t a = *reinterpret_cast<const f32x4_t*>(q0 + e);
+          x[e] = a[0]; x[e + 1] = a[1]; x[e + 2] = a[2]; x[e + 3] = a[3];
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < DPL; ++e) x[e] = q0[e];
+      }
+    } else {
+      const unsigned short* q0 = reinterpret_cast<const unsigned short*>(p.q) + row;
+      if (q_vec) {
+#pragma unroll
+        for (int e = 0; e < DPL; e += 4) {
+          const u32x2_t a = *reinterpret_cast<const u32x2_t*>(q0 + e);
+          x[e] = bf16_lo(a[0]); x[e + 1] = bf16_hi(a[0]); x[e + 2] = bf16_lo(a[1]); x[e + 3] = bf16_hi(a[1]);
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < DPL; ++e) x[e] = __uint_as_float((u32)q0[e] << 16);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < DPL; ++e) {
+      if constexpr (QUEST) {
+        qm[e] += fmaxf(x[e], 0.f);
+        qn[e] += fminf(x[e], 0.f);
+      } else {
+        qm[e] += x[e];
+      }
+    }
+  }
+  if constexpr (NS >= 4) {
+    float v[NS];
+#pragma unroll
+    for (int t = 0; t < NS; ++t)
+      v[t] = QUEST ? block_dot_quest<DPL, KBF16>(w1[t], w2[QUEST ? t : 0], qm, qn) : block_dot<DPL, KBF16>(w1[t], qm);
+    reduce_scatter16<NS>(v, lane);
+    constexpr int kCopies = 16 / NS;  // lanes holding each step
+    const int t = c16 / kCopies;
+    const int j = base + 16 * t + 4 * wave + r;
+    if (c16 % kCopies == 0 && j < p.nb_max) sc_row[j] = j < nb ? v[0] * p.score_scale : kNegInf;
+  } else {
+#pragma unroll
+    for (int t = 0; t < NS; ++t) {
+      const float a = QUEST ? block_score_quest<DPL, KBF16>(w1[t], w2[QUEST ? t : 0], qm, qn, p.score_scale)
+                            : block_score<DPL, KBF16>(w1[t], qm, p.score_scale);
+      const int j = base + 16 * t + 4 * wave + r;
+      if (c16 == 0 && j < p.nb_max) sc_row[j] = j < nb ? a : kNegInf;
+    }
+  }
+}
+
+// The rule on a stored score row, one workgroup per row: thread t holds the keys of
+// blocks t + 1024 e, e < KPT, in registers (KPT = 0: rows longer than 32 keys per thread are
+// read from memory in every pass).
+template <int KPT>
+__global__ __launch_bounds__(kSelThreads) void ia_condition_block_select_scores(SelectParams p) {
+  __shared__ TopkLds<kSelThreads> sel_lds;
+  const int h = blockIdx.x;
+  const int b = blockIdx.y;
+  const int bh = b * p.n_kv_heads + h;
+  const int seq_len = max(p.seq_lens[b], 0);
+  const int nb = min((seq_len + p.block_size - 1) / p.block_size, p.nb_max);
+  const float* sc_row = p.scores + (int64_t)bh * p.nb_max;
+  const int k_b = p.k_per_seq ? max(p.k_per_seq[b], 0) : p.k;
+  const TopkRule rule{p.forced_first, p.forced_last, k_b, p.forced_in_k, p.k_cap};
+  int32_t* out_idx = p.idx + (int64_t)bh * p.k_cap;
+  auto emit = [&](int pos, int j) { out_idx[pos] = j; };
+  int n;
+  if constexpr (KPT > 0) {
+    u32 key[KPT];
+#pragma unroll
+    for (int e = 0; e < KPT; ++e)  // (entries past the row's blocks hold -inf; past nb_max: unused)
+      key[e] = order_key(sc_row[min((int)threadIdx.x + kSelThreads * e, p.nb_max - 1)]);
+    n = topk_select_regs<kSelThreads, KPT>(sel_lds, key, nb, rule, emit);
+  } else {
+    n = topk_select<kSelThreads>(sel_lds, [&](int j) -> u32 { return order_key(sc_row[j]); }, nb, rule, emit);
+  }
+  if (threadIdx.x == 0) p.n_sel[bh] = n;
+}
+
+template <int D, bool KBF16, bool QUEST>
+void launch_scores(const SelectParams& p, int group, bool qf32, int batch, hipStream_t st) {
+  constexpr int kBlocks = ScoreShape<D, KBF16, QUEST>::kBlocks;
+  const dim3 grid((p.nb_max + kBlocks - 1) / kBlocks, p.n_kv_heads, batch);
+  // the query rows as vector loads where every row starts 16-byte aligned
+  const int64_t es = qf32 ? 4 : 2;
+  const int q_vec = reinterpret_cast<uintptr_t>(p.q) % 16 == 0 && p.q_batch_stride * es % 16 == 0 && p.q_row_stride * es % 16 == 0;
+  hipLaunchKernelGGL((ia_condition_block_scores<D, KBF16, QUEST>), grid, dim3(256), 0, st, p, group, qf32 ? 1 : 0, q_vec);
+}
+
+// p.scores set: score over the whole device, then select per row
+int run_two_launches(const SelectParams& p, int D, int group, bool qf32, bool kbf16, int batch, hipStream_t st) {
+  auto score = [&](auto d) {
+    constexpr int DD = decltype(d)::value;
+    if (p.quest) kbf16 ? launch_scores<DD, true, true>(p, group, qf32, batch, st)
+                       : launch_scores<DD, false, true>(p, group, qf32, batch, st);
+    else kbf16 ? launch_scores<DD, true, false>(p, group, qf32, batch, st)
+               : launch_scores<DD, false, false>(p, group, qf32, batch, st);
+  };
+  if (D == 128) score(std::integral_constant<int, 128>{});
+  else score(std::integral_constant<int, 64>{});
+  const int rc = check_launch("block scores");
+  if (rc) return rc;
+  const dim3 grid(p.n_kv_heads, batch);
+  auto select = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(kSelThreads), 0, st, p); };
+  const int per_thread = (p.nb_max + kSelThreads - 1) / kSelThreads;
+  if (per_thread <= 4) select(ia_condition_block_select_scores<4>);
+  else if (per_thread <= 8) select(ia_condition_block_select_scores<8>);
+  else if (per_thread <= 16) select(ia_condition_block_select_scores<16>);
+  else if (per_thread <= 32) select(ia_condition_block_select_scores<32>);
+  else select(ia_condition_block_select_scores<0>);
+  return check_launch("select_topk");
+}
+
 size_t select_ws_size(int batch, int hkv, int nb_max) {
   const size_t bh = (size_t)batch * hkv;
   return bh * (size_t)std::max(nb_max, 1) * 4;
@@ -210,7 +407,7 @@ size_t select_ws_size(int batch, int hkv, int nb_max) {
 
 template <int D, int G>
 int launch_select(const SelectParams& p, bool qf32, bool kbf16, dim3 grid, hipStream_t st) {
-  const size_t lds = (size_t)p.lds_scores * sizeof(float);
+  const size_t lds = (size_t)std::max(p.nb_max, 1) * sizeof(float);
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(kSelThreads), lds, st, p); };
   if (p.quest) {
     if (qf32) kbf16 ? go(ia_condition_block_select_topk<D, G, true, true, true>)
@@ -341,11 +538,21 @@ int ia_select_topk(const ia_decode_shape* shape, const void* q, const ia_block_k
   p.idx = idx;
   p.k_cap = k_cap;
   p.n_sel = n_sel;
-  // scores go to global memory when asked for, or when a row does not fit in LDS
-  p.scores = scores ? scores : (nb_max > kMaxLdsScores ? reinterpret_cast<float*>(workspace) : nullptr);
+  p.scores = scores;
   p.n_kv_heads = shape->n_kv_heads;
   p.score_scale = score_scale;
-  p.lds_scores = nb_max <= kMaxLdsScores ? nb_max : 0;
+  // Long rows in two launches, given memory for their scores.  The line: one workgroup
+  // streams its row's keys alone, and from the second key batch on (above 1024 blocks of
+  // bf16 D = 128) that costs more than a second launch.  One launch against two (graph
+  // replays, 8 kv heads): 8 rows of 1024 blocks 9.3 / 8.7 us, 2048 16.2 / 9.7, 4096 26.2 /
+  // 10.3, 15626 100.5 / 20.8, 32768 201 / 35.5; 128 rows of 1024 blocks 13.3 / 14.0, 2048
+  // 21.6 / 19.3, 4096 32.7 / 29.4.
+  float* stored = scores ? scores : (workspace && workspace_bytes >= need ? reinterpret_cast<float*>(workspace) : nullptr);
+  if (stored && nb_max > kOneLaunchBlocks) {
+    p.scores = stored;
+    return run_two_launches(p, D, G, shape->q_dtype == IA_F32, keys->dtype == IA_BF16, shape->batch,
+                            reinterpret_cast<hipStream_t>(stream));
+  }
   dim3 grid(shape->n_kv_heads, shape->batch);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const bool qf32 = shape->q_dtype == IA_F32;

@@ -264,6 +264,49 @@ __device__ __forceinline__ void topk_stage(TopkLds<NT>& L, u32 kmx, u32 kmn_inv)
   if (threadIdx.x == 0) L.n_tie = 0;
 }
 
+// The threshold pair among the in_bin <= kTieCands members of the threshold bucket listed
+// in L.tie_key / L.tie_idx (any order): a member's rank among them (key descending, then
+// index ascending: a strict order, so ranks are distinct); rank need - 1 is the threshold.
+// Every thread of the workgroup calls it after a barrier behind the list's writes.
+template <int NT>
+__device__ __forceinline__ void tie_threshold(TopkLds<NT>& L, int in_bin, int need, u32& kT, int& iT) {
+  if (in_bin <= 64) {
+    // every wave ranks the members from registers (lane i holds member i), so no
+    // LDS round trip per member and no barrier before the threshold is known
+    const int lane = threadIdx.x & 63;
+    const bool mem = lane < in_bin;
+    const u32 ki = mem ? L.tie_key[lane] : 0u;
+    const int ji = mem ? L.tie_idx[lane] : 0;
+    int rank = 0;
+    for (int e = 0; e < in_bin; ++e) {
+      const u32 ke = (u32)__builtin_amdgcn_readlane((int)ki, e);
+      const int je = __builtin_amdgcn_readlane(ji, e);
+      rank += (ke > ki || (ke == ki && je < ji)) ? 1 : 0;
+    }
+    const unsigned long long hit = __ballot(mem && rank == need - 1);
+    const int src = __ffsll((long long)hit) - 1;
+    kT = (u32)__builtin_amdgcn_readlane((int)ki, src);
+    iT = __builtin_amdgcn_readlane(ji, src);
+  } else {
+    for (int i = threadIdx.x; i < in_bin; i += NT) {
+      const u32 ki = L.tie_key[i];
+      const int ji = L.tie_idx[i];
+      int rank = 0;
+      for (int e = 0; e < in_bin; ++e) {
+        const u32 ke = L.tie_key[e];
+        rank += (ke > ki || (ke == ki && L.tie_idx[e] < ji)) ? 1 : 0;
+      }
+      if (rank == need - 1) {
+        L.thr_key = ki;
+        L.thr_idx = ji;
+      }
+    }
+    __syncthreads();
+    kT = L.thr_key;
+    iT = L.thr_idx;
+  }
+}
+
 // Every thread of the workgroup calls this (it synchronises, also on return).  key_at(j) returns
 // order_key(score_j) for 0 <= j < nb; emit(pos, j) is called for each chosen block,
 // pos = 0, 1, ... in ascending block order (only pos < k_cap).  Returns the number
@@ -334,43 +377,7 @@ __device__ __forceinline__ int topk_select(TopkLds<NT>& L, KeyAt key_at, int nb,
           }
         }
         __syncthreads();
-        // member i's rank among the bucket's members (key descending, then index
-        // ascending: a strict order, so ranks are distinct); rank need - 1 is the threshold
-        if (in_bin <= 64) {
-          // every wave ranks the members from registers (lane i holds member i), so no
-          // LDS round trip per member and no barrier before the threshold is known
-          const int lane = threadIdx.x & 63;
-          const bool mem = lane < in_bin;
-          const u32 ki = mem ? L.tie_key[lane] : 0u;
-          const int ji = mem ? L.tie_idx[lane] : 0;
-          int rank = 0;
-          for (int e = 0; e < in_bin; ++e) {
-            const u32 ke = (u32)__builtin_amdgcn_readlane((int)ki, e);
-            const int je = __builtin_amdgcn_readlane(ji, e);
-            rank += (ke > ki || (ke == ki && je < ji)) ? 1 : 0;
-          }
-          const unsigned long long hit = __ballot(mem && rank == need - 1);
-          const int src = __ffsll((long long)hit) - 1;
-          kT = (u32)__builtin_amdgcn_readlane((int)ki, src);
-          iT = __builtin_amdgcn_readlane(ji, src);
-        } else {
-          for (int i = threadIdx.x; i < in_bin; i += NT) {
-            const u32 ki = L.tie_key[i];
-            const int ji = L.tie_idx[i];
-            int rank = 0;
-            for (int e = 0; e < in_bin; ++e) {
-              const u32 ke = L.tie_key[e];
-              rank += (ke > ki || (ke == ki && L.tie_idx[e] < ji)) ? 1 : 0;
-            }
-            if (rank == need - 1) {
-              L.thr_key = ki;
-              L.thr_idx = ji;
-            }
-          }
-          __syncthreads();
-          kT = L.thr_key;
-          iT = L.thr_idx;
-        }
+        tie_threshold<NT>(L, in_bin, need, kT, iT);
       } else {
         fast = false;
       }
@@ -465,6 +472,175 @@ __device__ __forceinline__ int topk_select(TopkLds<NT>& L, KeyAt key_at, int nb,
   }
   __syncthreads();  // emitted entries (e.g. in LDS) are visible to the workgroup on return
   return min(base_sel, rule.k_cap);
+}
+
+// Places in block order for topk_select_regs: bit e of a thread's bits marks block t + NT e.
+// pre[e * waves + w] receives the marked blocks before wave w's part of stripe e (a scan
+// of the stripes' wave counts in block order); returns all marked blocks.  Every thread
+// calls it; two barriers.
+template <int NT, int KPT>
+__device__ __forceinline__ int stripe_prefix(u32 bits, int* pre) {
+  constexpr int kWv = NT / 64;
+  constexpr int kPer = (KPT * kWv + 63) / 64;  // counts per lane of the scan
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  int mine = 0;
+#pragma unroll
+  for (int e = 0; e < KPT; ++e) {
+    const int c = __popcll(__ballot(bits >> e & 1u));
+    if (lane == e) mine = c;
+  }
+  if (lane < KPT) pre[lane * kWv + wave] = mine;
+  __syncthreads();
+  int c[kPer], sum = 0;  // every wave scans all counts
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    c[i] = lane * kPer + i < KPT * kWv ? pre[lane * kPer + i] : 0;
+    sum += c[i];
+  }
+  const int inc = wave_inclusive_scan(sum);
+  __syncthreads();
+  if (wave == 0) {
+    int run = inc - sum;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      if (lane * kPer + i < KPT * kWv) pre[lane * kPer + i] = run;
+      run += c[i];
+    }
+  }
+  __syncthreads();
+  return __builtin_amdgcn_readlane(inc, 63);
+}
+
+// topk_select for a row whose keys the threads hold in registers: thread t owns blocks
+// t + NT e, e < KPT (KPT NT >= nb; the row is read once, coalesced), key[e] their order
+// keys (unused past nb).  The same rule, thresholds and order.
+template <int NT, int KPT, typename Emit>
+__device__ __forceinline__ int topk_select_regs(TopkLds<NT>& L, const u32 (&key)[KPT], int nb, const TopkRule& rule,
+                                                Emit emit) {
+  static_assert(KPT <= 32, "one bit per held key");
+  constexpr int kWv = NT / 64;
+  __shared__ int pre[KPT * kWv];
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  const TopkForced is_forced(rule, nb);
+  const TopkSizes sizes = topk_sizes(nb, rule);
+  const int k_eff = sizes.k_eff;
+  u32 cand = 0u, forced = 0u;
+#pragma unroll
+  for (int e = 0; e < KPT; ++e) {
+    const int j = threadIdx.x + NT * e;
+    if (j < nb) (is_forced(j) ? forced : cand) |= 1u << e;
+  }
+  auto each = [&](auto f) {
+#pragma unroll
+    for (int e = 0; e < KPT; ++e)
+      if (cand >> e & 1u) f(key[e], (int)threadIdx.x + NT * e);
+  };
+  u32 kT = 0u;
+  int iT = 0x7fffffff;
+  if (k_eff == 0) {
+    kT = 0xffffffffu;
+    iT = -1;
+  }
+  if (k_eff > 0 && k_eff < sizes.n_cand) {
+    u32 kmx = 0u, kmn_inv = 0u;
+    each([&](u32 k, int) {
+      kmx = max(kmx, k);
+      kmn_inv = max(kmn_inv, ~k);
+    });
+    topk_stage<NT>(L, kmx, kmn_inv);
+    __syncthreads();
+    kmx = 0u;
+    kmn_inv = 0u;
+#pragma unroll
+    for (int w = 0; w < kWv; ++w) {
+      kmx = max(kmx, L.red[0][w]);
+      kmn_inv = max(kmn_inv, L.red[1][w]);
+    }
+    const u32 kmn = ~kmn_inv;
+    const float fmax = key_value(kmx), fmin = key_value(kmn);
+    const float bscale = 256.f / (fmax - fmin);
+    bool fast = __builtin_isfinite(fmax) && __builtin_isfinite(fmin) && __builtin_isfinite(bscale) && bscale > 0.f;
+    auto bucket = [&](u32 k) { return min(255, (int)((key_value(k) - fmin) * bscale)); };
+    if (fast) {
+      each([&](u32 k, int) { atomicAdd(&L.hist[bucket(k)], 1u); });
+      __syncthreads();
+      int tb, need, in_bin;
+      threshold_bin_wave(L.hist, k_eff, tb, need, in_bin);
+      if (in_bin <= kTieCands) {
+        each([&](u32 k, int j) {
+          if (bucket(k) == tb) {
+            const int s = atomicAdd(&L.n_tie, 1);
+            L.tie_key[s] = k;
+            L.tie_idx[s] = j;
+          }
+        });
+        __syncthreads();
+        tie_threshold<NT>(L, in_bin, need, kT, iT);
+      } else {
+        fast = false;
+      }
+    }
+    if (!fast) {
+      __syncthreads();  // every wave is done with the bucket histogram
+      const u32 diff = kmx ^ kmn;
+      const int common_bytes = diff == 0u ? 4 : (__clz((int)diff) >> 3);
+      u32 prefix = 0u, mask = 0u;
+      if (common_bytes > 0) {
+        mask = common_bytes == 4 ? 0xffffffffu : ~(0xffffffffu >> (8 * common_bytes));
+        prefix = kmx & mask;
+      }
+      int remaining = k_eff, in_bin = sizes.n_cand;
+      for (int shift = 24 - 8 * common_bytes; shift >= 0; shift -= 8) {
+        for (int t = threadIdx.x; t < 256; t += NT) L.hist[t] = 0u;
+        __syncthreads();
+        each([&](u32 k, int) {
+          if ((k & mask) == prefix) atomicAdd(&L.hist[(k >> shift) & 255u], 1u);
+        });
+        __syncthreads();
+        if (wave == 0) threshold_bin<NT>(L, remaining);
+        __syncthreads();
+        const u32 digit = (u32)L.sh_int[1];
+        remaining = L.sh_int[2];
+        in_bin = L.sh_int[3];
+        prefix |= digit << shift;
+        mask |= 255u << shift;
+        __syncthreads();
+        if (remaining == in_bin) break;  // the whole bin is taken: the threshold is exact
+      }
+      kT = prefix;
+      if (remaining != in_bin) {  // the `remaining` lowest indices among keys equal to prefix
+        u32 eq = 0u;
+#pragma unroll
+        for (int e = 0; e < KPT; ++e)
+          if ((cand >> e & 1u) && key[e] == prefix) eq |= 1u << e;
+        stripe_prefix<NT, KPT>(eq, pre);
+#pragma unroll
+        for (int e = 0; e < KPT; ++e) {
+          const unsigned long long bal = __ballot(eq >> e & 1u);
+          if ((eq >> e & 1u) && pre[e * kWv + wave] + __popcll(bal & below) == remaining - 1)
+            L.thr_idx = threadIdx.x + NT * e;
+        }
+        __syncthreads();
+        iT = L.thr_idx;
+      }
+    }
+  }
+  u32 bits = forced;
+#pragma unroll
+  for (int e = 0; e < KPT; ++e)
+    if ((cand >> e & 1u) && (key[e] > kT || (key[e] == kT && (int)threadIdx.x + NT * e <= iT))) bits |= 1u << e;
+  __syncthreads();  // (the counts of a tie scan are read)
+  const int total = stripe_prefix<NT, KPT>(bits, pre);
+#pragma unroll
+  for (int e = 0; e < KPT; ++e) {
+    const unsigned long long bal = __ballot(bits >> e & 1u);
+    const int pos = pre[e * kWv + wave] + __popcll(bal & below);
+    if ((bits >> e & 1u) && pos < rule.k_cap) emit(pos, (int)threadIdx.x + NT * e);
+  }
+  return min(total, rule.k_cap);
 }
 
 }  // namespace ia
