@@ -375,6 +375,21 @@ IA_API int ia_fixed_mask_decode_fused(const ia_decode_shape* shape, const void* 
                                       size_t workspace_bytes, void* stream);
 
 /*
+ * ia_condition_decode_fused and (mask non-NULL: eps, term1_mass_exp and selected are
+ * not read) ia_fixed_mask_decode_fused for every GQA group they have an instance for:
+ * groups of 1, 2 and 4 as those two, and of 8 on bf16 caches or at head_dim 64.  The
+ * same workspace, semantics and results; ia_condition_one_launch_items is the fit
+ * query, 0 when the call does not fit one launch.  Replaces the same reference
+ * functions.
+ */
+IA_API int32_t ia_condition_one_launch_items(const ia_decode_shape* shape, const ia_block_summaries* sm,
+                                             int32_t kv_dtype, int32_t suffix_cap);
+IA_API int ia_condition_one_launch(const ia_decode_shape* shape, const void* q, const ia_block_summaries* sm,
+                                   const uint8_t* mask, const ia_paged_kv* prompt, const ia_suffix_kv* suffix,
+                                   float eps, int32_t term1_mass_exp, uint8_t* selected, float scale, void* out,
+                                   int32_t out_dtype, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Hybrid decode with an external per-(batch, kv head) block mask [batch, Hkv, nb]
  * uint8: representatives recomputed as q.k_bar/sqrt(D) + log(count), q and k_bar
  * rounded to bfloat16 for bfloat16 caches.

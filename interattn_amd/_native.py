@@ -190,6 +190,12 @@ SIGNATURES = {
         ctypes.c_int,
         [ctypes.POINTER(DecodeShape), _P, ctypes.POINTER(BlockSummaries), _P, ctypes.POINTER(PagedKV),
          ctypes.POINTER(SuffixKV), _F, _P, _I32, _P, _SZ, _P]),
+    "ia_condition_one_launch_items": (
+        ctypes.c_int32, [ctypes.POINTER(DecodeShape), ctypes.POINTER(BlockSummaries), _I32, _I32]),
+    "ia_condition_one_launch": (
+        ctypes.c_int,
+        [ctypes.POINTER(DecodeShape), _P, ctypes.POINTER(BlockSummaries), _P, ctypes.POINTER(PagedKV),
+         ctypes.POINTER(SuffixKV), _F, _I32, _P, _F, _P, _I32, _P, _SZ, _P]),
     "ia_fixed_mask_decode": (
         ctypes.c_int,
         [ctypes.POINTER(DecodeShape), _P, ctypes.POINTER(BlockSummaries), _P, ctypes.POINTER(PagedKV),

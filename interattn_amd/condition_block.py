@@ -322,9 +322,8 @@ def _suffix_desc(k_suffix, v_suffix, suffix_len_dev, prompt_dtype):
 
 
 def _one_launch():
-    """The condition rule's decode (``ia_condition_decode_fused``) and the fixed-mask
-    decode (``ia_fixed_mask_decode_fused``) run as one launch where the call fits one,
-    unless ``INTERATTN_CONDITION_ONE_LAUNCH=0`` asks for the multi-launch paths
+    """The condition rule's decode and the fixed-mask decode run as one launch
+    (``ia_condition_one_launch``) where the call fits one, unless ``INTERATTN_CONDITION_ONE_LAUNCH=0`` asks for the multi-launch paths
     (statistics, route, finalize, merge; route, finalize, merge)."""
     return os.environ.get("INTERATTN_CONDITION_ONE_LAUNCH", "1") != "0"
 
@@ -356,25 +355,20 @@ def _condition_decode(q_grouped, prompt_prefix, k_suffix, v_suffix, suffix_len_d
     if store_selected:
         selected = workspace_tensor(workspace, "selected_rows", (rows, nb), device=dev, dtype=torch.uint8)
     scale = head_dim ** -0.5
-    if mask is None and _one_launch() and lib.ia_condition_decode_fused_items(sh, sm, kv.dtype, sfx.cap) > 0:
+    if _one_launch() and lib.ia_condition_one_launch_items(sh, sm, kv.dtype, sfx.cap) > 0:
         # one launch: its workspace carries per-row counts from call to call (zero-filled
         # once, one per (heads, group, head_dim), whatever the prompt length and eps)
         fws = _scratch(workspace, ("condition_fused_scratch", n_kv_heads, group_size, head_dim),
                        lib.ia_condition_decode_fused_workspace_size(1, n_kv_heads, group_size, head_dim), dev)
-        rc = lib.ia_condition_decode_fused(sh, q.data_ptr(), sm, kv, sfx, float(eps), int(bool(term1_mass_exp)),
-                                           None if selected is None else selected.data_ptr(), scale,
-                                           out.data_ptr(), _code(output_dtype, "out"), fws.data_ptr(), fws.numel(),
-                                           _stream(q))
+        rc = lib.ia_condition_one_launch(sh, q.data_ptr(), sm, None if mask is None else mask.data_ptr(), kv, sfx,
+                                         float(eps), int(bool(term1_mass_exp)),
+                                         None if selected is None else selected.data_ptr(), scale, out.data_ptr(),
+                                         _code(output_dtype, "out"), fws.data_ptr(), fws.numel(), _stream(q))
     elif mask is None:
         ws = scratch()
         rc = lib.ia_condition_decode(sh, q.data_ptr(), sm, kv, sfx, float(eps), int(bool(term1_mass_exp)),
                                      None if selected is None else selected.data_ptr(), scale, out.data_ptr(),
                                      _code(output_dtype, "out"), ws.data_ptr(), ws.numel(), _stream(q))
-    elif _one_launch() and lib.ia_condition_decode_fused_items(sh, sm, kv.dtype, sfx.cap) > 0:
-        fws = _scratch(workspace, ("condition_fused_scratch", n_kv_heads, group_size, head_dim),
-                       lib.ia_condition_decode_fused_workspace_size(1, n_kv_heads, group_size, head_dim), dev)
-        rc = lib.ia_fixed_mask_decode_fused(sh, q.data_ptr(), sm, mask.data_ptr(), kv, sfx, scale, out.data_ptr(),
-                                            _code(output_dtype, "out"), fws.data_ptr(), fws.numel(), _stream(q))
     else:
         ws = scratch()
         rc = lib.ia_fixed_mask_decode(sh, q.data_ptr(), sm, mask.data_ptr(), kv, sfx, scale, out.data_ptr(),

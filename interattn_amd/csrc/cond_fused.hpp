@@ -28,7 +28,7 @@ namespace ia {
 
 template <int D, int G>
 struct CondLds {
-  float s[G][kCondItemBlocks];       // s per (query row, own block); then the representatives' weights
+  alignas(16) float s[G][kCondItemBlocks];  // s per (query row, own block); then the representatives' weights
   float dl[G][kCondItemBlocks];      // delta per (query row, own block)
   float lc[kCondItemBlocks];         // log(valid tokens) per own block, -inf for an empty one
   float part[kMaxItemsPerBh][4][G];  // the row's items' partials (z_m, z_l, c_m, c_l) per query row

@@ -866,10 +866,17 @@ CondFusedWs cond_fused_ws_layout(int batch, int hkv, int g, int d) {
 // 0 when the call does not fit one launch: every row's items must be resident at
 // once (they exchange their statistics), an item owns at most kCondItemBlocks
 // blocks and its selected blocks plus the suffix must fit the finalize's LDS lists.
-int cond_fused_items(int batch, int hkv, int g, int d, int nb, int block_size, int sfx_cap, int kv_dtype,
-                     bool q_f32, hipStream_t st) {
-  if (g > 4 || (d != 64 && d != 128) || nb <= 0 || nb > 65535 || batch <= 0) return 0;
+// max_group: the caller's bound on the GQA group (groups of 8 came later than the entry
+// points that refuse them).  G = 8, one launch against four (graph replays, batch 1 x 8 kv
+// heads, D = 128, 64-token blocks): 20K tokens 24.8 / 40.6 us (bf16 summaries 24.5 / 36.9),
+// 128K 30.1 / 44.3, fixed mask 22.1 / 41.5 and 24.9 / 37.7 us; never slower over 4K-128K,
+// 16-token blocks, 30% selected and 600-token suffixes.  It is the latency chain of the
+// smaller groups with twice the statistics per block and twice the merge.
+int cond_fused_items(int max_group, int batch, int hkv, int g, int d, int nb, int block_size, int sfx_cap,
+                     int kv_dtype, bool q_f32, hipStream_t st) {
+  if ((d != 64 && d != 128) || nb <= 0 || nb > 65535 || batch <= 0) return 0;
   if (kv_dtype != IA_BF16 && kv_dtype != IA_F32) return 0;
+  if (g > max_group || (g > 4 && d == 128 && kv_dtype == IA_F32)) return 0;  // (the latter: no instance)
   if ((kv_dtype == IA_F32) != q_f32) return 0;
   DecodeParams probe{};
   probe.q_f32 = q_f32;
@@ -894,7 +901,7 @@ int cond_fused_items(int batch, int hkv, int g, int d, int nb, int block_size, i
   return (int)n;
 }
 
-int run_condition_fused(const uint8_t* mask, const ia_decode_shape* shape, const void* q,
+int run_condition_fused(int max_group, const uint8_t* mask, const ia_decode_shape* shape, const void* q,
                         const ia_block_summaries* sm, const ia_paged_kv* prompt, const ia_suffix_kv* sfx, float eps,
                         int32_t mass_exp, uint8_t* selected, float scale, void* out, int32_t out_dtype,
                         void* workspace, size_t workspace_bytes, void* stream) {
@@ -927,7 +934,7 @@ int run_condition_fused(const uint8_t* mask, const ia_decode_shape* shape, const
     return fail(IA_ERR_WORKSPACE, "workspace must be 256-byte aligned");
   if (shape->batch == 0) return IA_OK;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const int n_it = cond_fused_items(shape->batch, shape->n_kv_heads, G, D, sm->nb, sm->block_size, sfx_cap,
+  const int n_it = cond_fused_items(max_group, shape->batch, shape->n_kv_heads, G, D, sm->nb, sm->block_size, sfx_cap,
                                     prompt->dtype, shape->q_dtype == IA_F32, st);
   if (n_it <= 0)
     return fail(IA_ERR_UNSUPPORTED, "this condition call does not fit one launch; use ia_condition_decode");
@@ -1002,16 +1009,32 @@ size_t ia_condition_decode_fused_workspace_size(int32_t batch, int32_t n_kv_head
 int32_t ia_condition_decode_fused_items(const ia_decode_shape* shape, const ia_block_summaries* sm,
                                         int32_t kv_dtype, int32_t suffix_cap) {
   if (ia::check_shape(shape) || !sm) return 0;
-  return ia::cond_fused_items(shape->batch, shape->n_kv_heads, shape->n_q_heads / shape->n_kv_heads,
+  return ia::cond_fused_items(4, shape->batch, shape->n_kv_heads, shape->n_q_heads / shape->n_kv_heads,
                               shape->head_dim, sm->nb, sm->block_size, suffix_cap, kv_dtype,
                               shape->q_dtype == IA_F32, nullptr);
+}
+
+int32_t ia_condition_one_launch_items(const ia_decode_shape* shape, const ia_block_summaries* sm, int32_t kv_dtype,
+                                      int32_t suffix_cap) {
+  if (ia::check_shape(shape) || !sm) return 0;
+  return ia::cond_fused_items(8, shape->batch, shape->n_kv_heads, shape->n_q_heads / shape->n_kv_heads,
+                              shape->head_dim, sm->nb, sm->block_size, suffix_cap, kv_dtype,
+                              shape->q_dtype == IA_F32, nullptr);
+}
+
+int ia_condition_one_launch(const ia_decode_shape* shape, const void* q, const ia_block_summaries* sm,
+                            const uint8_t* mask, const ia_paged_kv* prompt, const ia_suffix_kv* suffix, float eps,
+                            int32_t term1_mass_exp, uint8_t* selected, float scale, void* out, int32_t out_dtype,
+                            void* workspace, size_t workspace_bytes, void* stream) {
+  return ia::run_condition_fused(8, mask, shape, q, sm, prompt, suffix, mask ? 0.f : eps, mask ? 0 : term1_mass_exp,
+                                 selected, scale, out, out_dtype, workspace, workspace_bytes, stream);
 }
 
 int ia_condition_decode_fused(const ia_decode_shape* shape, const void* q, const ia_block_summaries* sm,
                               const ia_paged_kv* prompt, const ia_suffix_kv* suffix, float eps,
                               int32_t term1_mass_exp, uint8_t* selected, float scale, void* out, int32_t out_dtype,
                               void* workspace, size_t workspace_bytes, void* stream) {
-  return ia::run_condition_fused(nullptr, shape, q, sm, prompt, suffix, eps, term1_mass_exp, selected, scale, out,
+  return ia::run_condition_fused(4, nullptr, shape, q, sm, prompt, suffix, eps, term1_mass_exp, selected, scale, out,
                                  out_dtype, workspace, workspace_bytes, stream);
 }
 
@@ -1020,7 +1043,7 @@ int ia_fixed_mask_decode_fused(const ia_decode_shape* shape, const void* q, cons
                                float scale, void* out, int32_t out_dtype, void* workspace, size_t workspace_bytes,
                                void* stream) {
   if (!mask) return ia::fail(IA_ERR_INVALID, "fixed-mask decode needs a mask");
-  return ia::run_condition_fused(mask, shape, q, sm, prompt, suffix, 0.f, 0, nullptr, scale, out, out_dtype,
+  return ia::run_condition_fused(4, mask, shape, q, sm, prompt, suffix, 0.f, 0, nullptr, scale, out, out_dtype,
                                  workspace, workspace_bytes, stream);
 }
 

@@ -20,12 +20,12 @@ int run_f32(const DecodeParams& p, int src, dim3 grid, hipStream_t st, int* resi
     case kSrcTopkFused:
       if (resident) return *resident = resident_wgs<D, G, KvF32, kSrcTopkFused>(), IA_OK;
       return launch_paged_finalize<D, G, KvF32, kSrcTopkFused>(p, grid, st);
-    case kSrcCondFused:  // the one-launch condition call runs groups of up to 4 query rows
-      if constexpr (G <= 4) {
+    case kSrcCondFused:  // (groups of 8 at D = 128 need more registers than two waves per SIMD have)
+      if constexpr (G <= 4 || D == 64) {
         if (resident) return *resident = resident_wgs<D, G, KvF32, kSrcCondFused>(), IA_OK;
         return launch_paged_finalize<D, G, KvF32, kSrcCondFused>(p, grid, st);
       } else {
-        return fail(IA_ERR_UNSUPPORTED, "one-launch condition call: GQA group above 4");
+        return fail(IA_ERR_UNSUPPORTED, "one-launch condition call: fp32 caches with a GQA group of 8 at head_dim 128");
       }
   }
   return fail(IA_ERR_UNSUPPORTED, "unit source");

@@ -782,7 +782,10 @@ __global__ __launch_bounds__(kFinThreads, 2) void ia_condition_block_paged_final
   // and top-k-list sources never.
   constexpr bool kKeyLdsAny =
       kMfma && kBf16 && D == 128 && ((SRC == kSrcTopkFused && KROWS) || SRC == kSrcLists || SRC == kSrcCondFused);
-  __shared__ u32x4_t key_lds[kKeyLdsAny ? kFinWaves : 1][kKeyLdsAny ? 256 : 1];
+  // (the one-launch condition call at G = 8 takes the place of its prologue's statistics,
+  // which are dead by then and as large: 145 KiB of LDS instead of 177)
+  constexpr bool kKeyOnStats = kKeyLdsAny && SRC == kSrcCondFused && G == 8;
+  __shared__ u32x4_t key_lds[kKeyLdsAny && !kKeyOnStats ? kFinWaves : 1][kKeyLdsAny && !kKeyOnStats ? 256 : 1];
   __shared__ float q_lds[kQLds ? G * D : 1];
   __shared__ float wm_lds[kFinWaves][G];
   __shared__ float wl_lds[kFinWaves][G];
@@ -1489,7 +1492,13 @@ __global__ __launch_bounds__(kFinThreads, 2) void ia_condition_block_paged_final
       // sw(t) = t the reads of lanes c16 and c16 + 2 met in one group)
       u32x4_t kop[kKeyLds ? kMfmaK : 1];
       if constexpr (kKeyLds) {
-        u32x4_t* kl = key_lds[wave];
+        u32x4_t* kl = key_lds[0];
+        if constexpr (kKeyOnStats) {
+          static_assert(sizeof(cond_lds.s) + sizeof(cond_lds.dl) >= kFinWaves * 256 * sizeof(u32x4_t), "key slots");
+          kl = reinterpret_cast<u32x4_t*>(&cond_lds.s[0][0]) + 256 * wave;
+        } else {
+          kl = key_lds[wave];
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int t = 4 * i + r;
