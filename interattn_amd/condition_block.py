@@ -109,15 +109,9 @@ _summary_storage_dtypes = summary_storage_dtypes
 
 def _kv_desc(k_block, v_block, block_size):
     """Describe ``[Hkv, nb, B, D]`` prompt views as a pool of ``nb`` pages of ``B`` tokens."""
-    kv = N.PagedKV()
-    kv.k = k_block.data_ptr()
-    kv.v = v_block.data_ptr()
-    kv.dtype = _code(k_block.dtype, "prompt K/V")
-    kv.page_size = int(block_size)
-    kv.n_pages = int(k_block.shape[1])
-    kv.k_page_stride, kv.k_head_stride, kv.k_token_stride = int(k_block.stride(1)), int(k_block.stride(0)), int(k_block.stride(2))
-    kv.v_page_stride, kv.v_head_stride, kv.v_token_stride = int(v_block.stride(1)), int(v_block.stride(0)), int(v_block.stride(2))
-    return kv
+    ks, vs = k_block.stride(), v_block.stride()
+    return N.PagedKV(k_block.data_ptr(), v_block.data_ptr(), _code(k_block.dtype, "prompt K/V"), int(block_size),
+                     k_block.shape[1], ks[1], ks[0], ks[2], vs[1], vs[0], vs[2])
 
 
 def _build_prompt_blocks(k_all, v_all, block_size, *, summary_dtype=None, mixed=None, k_bar_dtype=None):
@@ -185,15 +179,12 @@ def _build_prompt_blocks(k_all, v_all, block_size, *, summary_dtype=None, mixed=
 
 def _summaries_desc(prefix, n_kv_heads, head_dim):
     """C-ABI view of a prefix dict (contiguous summary arrays, int32 counts)."""
-    sm = N.BlockSummaries()
     keep = []
 
-    def arr(name, required=True):
+    def arr(name):
         t = prefix.get(name)
         if t is None:
-            if required:
-                raise ValueError(f"prompt prefix lacks {name!r}")
-            return None
+            raise ValueError(f"prompt prefix lacks {name!r}")
         if not t.is_contiguous():
             t = t.contiguous()
         keep.append(t)
@@ -201,7 +192,7 @@ def _summaries_desc(prefix, n_kv_heads, head_dim):
 
     k_bar, v_bar = arr("k_bar"), arr("v_bar")
     nb = int(k_bar.shape[-2])
-    if tuple(k_bar.shape) != (n_kv_heads, nb, head_dim):
+    if k_bar.shape != (n_kv_heads, nb, head_dim):
         raise ValueError(f"k_bar must be [Hkv, nb, D] = {(n_kv_heads, nb, head_dim)}, got {tuple(k_bar.shape)}")
     bounds = prefix.get("k_bounds")
     if bounds is not None:
@@ -210,7 +201,6 @@ def _summaries_desc(prefix, n_kv_heads, head_dim):
             raise ValueError(f"k_bounds must be contiguous [Hkv, nb, 2D] = {(n_kv_heads, nb, 2 * head_dim)}")
         keep.append(bounds)
         k_max = k_min = bounds
-        sm.bounds_packed = 1
     else:
         k_max, k_min = arr("k_max"), arr("k_min")
         if k_max.dtype != k_min.dtype:
@@ -223,13 +213,13 @@ def _summaries_desc(prefix, n_kv_heads, head_dim):
     vnm, vna = arr("v_norm_max"), arr("v_norm_all")
     if vnm.dtype != torch.float32 or vna.dtype != torch.float32:
         raise ValueError("v_norm_max and v_norm_all must be float32")
-    sm.k_bar, sm.k_max, sm.k_min, sm.v_bar = k_bar.data_ptr(), k_max.data_ptr(), k_min.data_ptr(), v_bar.data_ptr()
-    sm.k_bar_dtype = _code(k_bar.dtype, "k_bar")
-    sm.bounds_dtype = _code(k_max.dtype, "k_max")
-    sm.v_bar_dtype = _code(v_bar.dtype, "v_bar")
-    sm.v_norm_max, sm.v_norm_all, sm.counts = vnm.data_ptr(), vna.data_ptr(), counts.data_ptr()
-    sm.nb = nb
-    sm.block_size = int(prefix.get("_block_size", prefix["k_block_attn"].shape[2]))
+    block_size = prefix.get("_block_size")
+    if block_size is None:
+        block_size = prefix["k_block_attn"].shape[2]
+    sm = N.BlockSummaries(k_bar.data_ptr(), k_max.data_ptr(), k_min.data_ptr(), v_bar.data_ptr(),
+                          _code(k_bar.dtype, "k_bar"), _code(k_max.dtype, "k_max"), _code(v_bar.dtype, "v_bar"),
+                          vnm.data_ptr(), vna.data_ptr(), counts.data_ptr(), nb, int(block_size),
+                          0 if bounds is None else 1)
     return sm, keep, nb
 
 
@@ -241,13 +231,10 @@ def _grouped_shape(q_grouped):
     q = q_grouped.reshape(rows, head_dim)
     if q.stride(1) != 1:
         q = q.contiguous()
-    sh = N.DecodeShape()
-    sh.batch, sh.n_q_heads, sh.n_kv_heads, sh.head_dim = 1, rows, n_kv_heads, head_dim
-    sh.q_batch_stride, sh.q_row_stride = int(q.stride(0)) * rows, int(q.stride(0))
     if q.dtype not in (torch.float32, torch.bfloat16):
         raise ValueError("q must be float32 or bfloat16")
-    sh.q_dtype = _code(q.dtype, "q")
-    return q, sh
+    row = q.stride(0)
+    return q, N.DecodeShape(1, rows, n_kv_heads, head_dim, row * rows, row, _code(q.dtype, "q"))
 
 
 # ------------------------------------------------------------------ selection
@@ -302,22 +289,18 @@ def _select_prompt_blocks_triton(q_grouped, prefix, eps, term1_mass_exp=False):
 # ------------------------------------------------------------------ fused decode
 
 def _suffix_desc(k_suffix, v_suffix, suffix_len_dev, prompt_dtype):
-    sfx = N.SuffixKV()
     if k_suffix is None or k_suffix.shape[1] == 0:
-        return sfx, []
+        return N.SuffixKV(), []
     _require_cuda(k_suffix, v_suffix, suffix_len_dev)
     if k_suffix.dtype != prompt_dtype or v_suffix.dtype != prompt_dtype:
         raise ValueError("suffix K/V must have the prompt K/V dtype")
-    if k_suffix.stride(2) != 1 or v_suffix.stride(2) != 1:
+    ks, vs = k_suffix.stride(), v_suffix.stride()
+    if ks[2] != 1 or vs[2] != 1:
         raise ValueError("suffix rows must be contiguous")
     if suffix_len_dev.dtype != torch.int32 or suffix_len_dev.numel() != 1:
         raise ValueError("suffix_len_dev must be one int32 on the device")
-    sfx.k, sfx.v = k_suffix.data_ptr(), v_suffix.data_ptr()
-    sfx.k_batch_stride, sfx.k_head_stride, sfx.k_token_stride = 0, int(k_suffix.stride(0)), int(k_suffix.stride(1))
-    sfx.v_batch_stride, sfx.v_head_stride, sfx.v_token_stride = 0, int(v_suffix.stride(0)), int(v_suffix.stride(1))
-    sfx.len = suffix_len_dev.data_ptr()
-    sfx.len_stride = 0
-    sfx.cap = int(k_suffix.shape[1])
+    sfx = N.SuffixKV(k_suffix.data_ptr(), v_suffix.data_ptr(), 0, ks[0], ks[1], 0, vs[0], vs[1],
+                     suffix_len_dev.data_ptr(), 0, k_suffix.shape[1])
     return sfx, [k_suffix, v_suffix, suffix_len_dev]
 
 
@@ -358,8 +341,11 @@ def _condition_decode(q_grouped, prompt_prefix, k_suffix, v_suffix, suffix_len_d
     if _one_launch() and lib.ia_condition_one_launch_items(sh, sm, kv.dtype, sfx.cap) > 0:
         # one launch: its workspace carries per-row counts from call to call (zero-filled
         # once, one per (heads, group, head_dim), whatever the prompt length and eps)
-        fws = _scratch(workspace, ("condition_fused_scratch", n_kv_heads, group_size, head_dim),
-                       lib.ia_condition_decode_fused_workspace_size(1, n_kv_heads, group_size, head_dim), dev)
+        key = ("condition_fused_scratch", n_kv_heads, group_size, head_dim)
+        fws = None if workspace is None else workspace.get(key)
+        if fws is None or fws.device != dev:
+            fws = _scratch(workspace, key,
+                           lib.ia_condition_decode_fused_workspace_size(1, n_kv_heads, group_size, head_dim), dev)
         rc = lib.ia_condition_one_launch(sh, q.data_ptr(), sm, None if mask is None else mask.data_ptr(), kv, sfx,
                                          float(eps), int(bool(term1_mass_exp)),
                                          None if selected is None else selected.data_ptr(), scale, out.data_ptr(),

@@ -34,7 +34,9 @@ def _code(dtype, what):
 
 
 def _stream(t):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The raw handle of torch's current stream on ``t``'s device (without building a
+    ``torch.cuda.Stream`` object, which took 2 us of a call's 19 us on the host)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _require_cuda(*tensors):
@@ -48,20 +50,18 @@ def workspace_tensor(workspace, key, shape, *, device, dtype, zero=False):
 
     Mirrors ``_workspace_empty`` (CBT/core.py:558-570); ``zero=True`` zero-fills a new
     tensor."""
-    shape = tuple(int(s) for s in shape)
+    t = None if workspace is None else workspace.get(key)
+    if t is not None and t.shape == tuple(shape) and t.dtype == dtype and t.device == device:
+        return t
     make = torch.zeros if zero else torch.empty
-    if workspace is None:
-        return make(shape, device=device, dtype=dtype)
-    t = workspace.get(key)
-    if t is None or tuple(t.shape) != shape or t.device != device or t.dtype != dtype:
-        t = make(shape, device=device, dtype=dtype)
+    t = make(tuple(int(s) for s in shape), device=device, dtype=dtype)
+    if workspace is not None:
         workspace[key] = t
     return t
 
 
 def _scratch(workspace, key, nbytes, device):
-    t = workspace_tensor(workspace, key, (max(int(nbytes), 1),), device=device, dtype=torch.uint8, zero=True)
-    return t
+    return workspace_tensor(workspace, key, (max(int(nbytes), 1),), device=device, dtype=torch.uint8, zero=True)
 
 
 def _check_i32(t, name, shape=None):
@@ -74,32 +74,27 @@ def _check_i32(t, name, shape=None):
 def paged_kv(pool_k, pool_v, block_table=None, scales=None):
     """Describe a pool for the C ABI.  Returns ``(PagedKV, keepalive)``."""
     _require_cuda(pool_k, pool_v, block_table)
-    if pool_k.dim() != 4 or pool_v.dim() != 4 or pool_k.shape != pool_v.shape:
+    shape = pool_k.shape
+    if len(shape) != 4 or shape != pool_v.shape:
         raise ValueError("pool_k/pool_v must both be [n_pages, Hkv, page_size, D]")
     if pool_k.dtype != pool_v.dtype:
         raise ValueError("pool_k and pool_v must share a dtype")
-    if pool_k.stride(3) != 1 or pool_v.stride(3) != 1:
+    ks_, vs_ = pool_k.stride(), pool_v.stride()
+    if ks_[3] != 1 or vs_[3] != 1:
         raise ValueError("pool rows (last dim) must be contiguous")
     code = _code(pool_k.dtype, "pool")
-    n_pages, hkv, page, d = pool_k.shape
-    kv = N.PagedKV()
-    kv.k = pool_k.data_ptr()
-    kv.v = pool_v.data_ptr()
-    kv.dtype = code
-    kv.page_size = int(page)
-    kv.n_pages = int(n_pages)
-    kv.k_page_stride, kv.k_head_stride, kv.k_token_stride = (int(s) for s in pool_k.stride()[:3])
-    kv.v_page_stride, kv.v_head_stride, kv.v_token_stride = (int(s) for s in pool_v.stride()[:3])
+    n_pages, hkv, page, _ = shape
     keep = [pool_k, pool_v]
+    table = (None, 0, 0)  # block_table, bt_stride, bt_cols
     if block_table is not None:
         _check_i32(block_table, "block_table")
         if block_table.dim() != 2 or block_table.stride(1) != 1:
             raise ValueError("block_table must be [batch, max_pages] with contiguous rows")
-        kv.block_table = block_table.data_ptr()
-        kv.bt_stride = int(block_table.stride(0)) if block_table.shape[0] > 1 else int(block_table.shape[1])
-        kv.bt_stride = max(kv.bt_stride, 1)
-        kv.bt_cols = int(block_table.shape[1])
+        rows, cols = block_table.shape
+        table = (block_table.data_ptr(), max(block_table.stride(0) if rows > 1 else cols, 1), cols)
         keep.append(block_table)
+    kv = N.PagedKV(pool_k.data_ptr(), pool_v.data_ptr(), code, page, n_pages, ks_[0], ks_[1], ks_[2], vs_[0], vs_[1],
+                   vs_[2], *table)
     if code == N.IA_FP8_E4M3:
         if scales is None:
             raise ValueError("fp8 pools need scales=(k_scale, v_scale), each [n_pages, Hkv] float32")
@@ -153,22 +148,15 @@ def sequence_scales(scales, block_table):
 
 
 def _decode_shape(q, hkv):
-    if q.dim() != 3 or q.stride(2) != 1:
+    stride = q.stride()
+    if len(stride) != 3 or stride[2] != 1:
         raise ValueError("q must be [batch, n_q_heads, D] with contiguous rows")
     b, hq, d = q.shape
     if hq % hkv != 0:
         raise ValueError("n_q_heads must be a multiple of n_kv_heads (grouped query attention)")
-    sh = N.DecodeShape()
-    sh.batch = int(b)
-    sh.n_q_heads = int(hq)
-    sh.n_kv_heads = int(hkv)
-    sh.head_dim = int(d)
-    sh.q_batch_stride = int(q.stride(0))
-    sh.q_row_stride = int(q.stride(1))
     if q.dtype not in (torch.float32, torch.bfloat16):
         raise ValueError("q must be float32 or bfloat16")
-    sh.q_dtype = _code(q.dtype, "q")
-    return sh
+    return N.DecodeShape(b, hq, hkv, d, stride[0], stride[1], _DTYPE_CODE[q.dtype])
 
 
 # --------------------------------------------------------------------------- summaries
@@ -278,20 +266,15 @@ def _block_keys(k_bar, score):
         raise ValueError("score='quest' takes k_bar=(k_max, k_min)")
     ref = arrays[0]
     _require_cuda(*arrays)
+    shape, stride, dtype = ref.shape, ref.stride(), ref.dtype
     for t in arrays:
         if t.dim() != 4 or t.stride(3) != 1 or t.stride(2) != t.shape[3]:
             raise ValueError("block keys must be [B, Hkv, nb_max, D] with contiguous blocks")
-        if t.shape != ref.shape or t.stride() != ref.stride() or t.dtype != ref.dtype:
+        if t is not ref and (t.shape != shape or t.stride() != stride or t.dtype != dtype):
             raise ValueError("k_max and k_min must share shape, strides and dtype")
-    keys = N.BlockKeys()
-    keys.score = SCORES[score]
-    keys.dtype = _code(ref.dtype, "block keys")
-    if score == "quest":
-        keys.k_max, keys.k_min = arrays[0].data_ptr(), arrays[1].data_ptr()
-    else:
-        keys.k_bar = ref.data_ptr()
-    keys.batch_stride, keys.head_stride = int(ref.stride(0)), int(ref.stride(1))
-    return keys, tuple(int(x) for x in ref.shape), ref.dtype, arrays
+    code = _code(dtype, "block keys")
+    ptrs = (None, ref.data_ptr(), arrays[1].data_ptr()) if score == "quest" else (ref.data_ptr(), None, None)
+    return N.BlockKeys(SCORES[score], code, *ptrs, stride[0], stride[1]), shape, dtype, arrays
 
 
 def set_wait_limit(ticks):
@@ -367,8 +350,8 @@ def select_blocks_topk(q, k_bar, seq_lens, k, *, block_size, forced_first=0, for
 def _out_tensor(q, out, out_dtype, workspace):
     dtype = q.dtype if out_dtype is None else out_dtype
     if out is None:
-        out = workspace_tensor(workspace, "attention_output", tuple(q.shape), device=q.device, dtype=dtype)
-    if tuple(out.shape) != tuple(q.shape) or not out.is_contiguous():
+        out = workspace_tensor(workspace, "attention_output", q.shape, device=q.device, dtype=dtype)
+    if out.shape != q.shape or not out.is_contiguous():
         raise ValueError("out must be a contiguous [batch, n_q_heads, D] tensor")
     if out.dtype not in (torch.float32, torch.bfloat16):
         raise ValueError("out must be float32 or bfloat16")
@@ -580,11 +563,13 @@ def sparse_topk_decode(q, pool_k, pool_v, block_table, seq_lens, k_bar, k, *, bl
         n_sel = workspace_tensor(workspace, "topk_n_sel", (b, hkv), device=dev, dtype=torch.int32)
     lib = N.lib()
     g = int(q.shape[1]) // hkv
-    ws_bytes = lib.ia_sparse_topk_decode_workspace_size(b, hkv, g, d, nb_max, k_cap, int(block_size))
     # the launch keeps per-row counts in its workspace from call to call: one
-    # zero-filled buffer per call shape
-    ws = _scratch(workspace if workspace is not None else {},
-                  ("topk_decode_scratch", b, hkv, g, d, nb_max, k_cap, int(block_size)), ws_bytes, dev)
+    # zero-filled buffer per call shape (whose size it therefore fixes)
+    key = ("topk_decode_scratch", b, hkv, g, d, nb_max, k_cap, int(block_size))
+    ws = None if workspace is None else workspace.get(key)
+    if ws is None or ws.device != dev:
+        ws = _scratch(workspace, key,
+                      lib.ia_sparse_topk_decode_workspace_size(b, hkv, g, d, nb_max, k_cap, int(block_size)), dev)
     rc = lib.ia_sparse_topk_decode(
         sh, q.data_ptr(), kv, seq_lens.data_ptr(), keys, int(block_size), nb_max, int(k),
         None if k_per_seq is None else k_per_seq.data_ptr(), int(forced_first), int(forced_last),
