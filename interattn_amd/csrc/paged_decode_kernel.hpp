@@ -778,10 +778,13 @@ __global__ __launch_bounds__(kFinThreads, 2) void ia_condition_block_paged_final
   // condition calls' few-subtile items).  Where every workgroup streams equal shares
   // at the HBM rate the transpose costs more than it gains (C4 +0.66 us), so the
   // one-launch top-k call takes it in its KROWS instance only (the host picks that
-  // one for launches with per-sequence k, its variable-length batches), and the dense
-  // and top-k-list sources never.
+  // one for launches with per-sequence k, its variable-length batches).  The dense source
+  // takes it with a ring of 2 (its consume is then the longer part of a step): 8 ragged
+  // sequences of 4-12K tokens 60.6 -> 56.8 us, 32 of 1-2K 42.5 -> 38.6, 16 x 64K 650 ->
+  // 639, one of 32K 30.2 / 30.4 (with a ring of 3: 58.1, 39.5, 640 and 30.8).  The
+  // top-k-list source never does.
   constexpr bool kKeyLdsAny =
-      kMfma && kBf16 && D == 128 && ((SRC == kSrcTopkFused && KROWS) || SRC == kSrcLists || SRC == kSrcCondFused);
+      kMfma && kBf16 && D == 128 && ((SRC == kSrcTopkFused && KROWS) || SRC == kSrcLists || SRC == kSrcCondFused || SRC == kSrcDense);
   // (the one-launch condition call at G = 8 takes the place of its prologue's statistics,
   // which are dead by then and as large: 145 KiB of LDS instead of 177)
   constexpr bool kKeyOnStats = kKeyLdsAny && SRC == kSrcCondFused && G == 8;
@@ -1346,11 +1349,12 @@ __global__ __launch_bounds__(kFinThreads, 2) void ia_condition_block_paged_final
   // issue: a load issued by consume would make the wave wait for every load in
   // flight (the vector memory counter drains in order).
   auto stream = [&](auto&& issue, auto&& consume) {
-    // The one-launch top-k call's long streams whose consume is the longer one (keys
-    // through LDS, fp8 codes widened) keep one subtile in flight per wave: a CU then
-    // streams faster than with two (C3 -1.0 to -1.2 us, C5 -1.2 us; same bits).  The
-    // condition-rule calls' short streams keep the deeper ring for their start.
-    constexpr int NBUF = (SRC == kSrcTopkFused && (KROWS || kFp8)) ? 2 : KV::kRing;
+    // The one-launch top-k call's and the dense source's long streams whose consume is the
+    // longer one (keys through LDS, fp8 codes widened) keep one subtile in flight per wave:
+    // a CU then streams faster than with two (C3 -1.0 to -1.2 us, C5 -1.2 us, dense fp8 8
+    // x 4-12K 37.9 -> 36.5 us; same bits).  The condition-rule calls' short streams keep
+    // the deeper ring for their start.
+    constexpr int NBUF = (SRC == kSrcTopkFused && (KROWS || kFp8)) || (SRC == kSrcDense && (kKeyLdsAny || kFp8)) ? 2 : KV::kRing;
     // the priority feedback below stays in the fp8 and key-row top-k calls (measured
     // faster with it) and in the finalizes of the multi-launch paths; the uniform bf16
     // top-k call (C4 -0.4, C2 -0.15 us) and the one-launch condition calls (-0.1 to
