@@ -781,10 +781,11 @@ __global__ __launch_bounds__(kFinThreads, 2) void ia_condition_block_paged_final
   // one for launches with per-sequence k, its variable-length batches).  The dense source
   // takes it with a ring of 2 (its consume is then the longer part of a step): 8 ragged
   // sequences of 4-12K tokens 60.6 -> 56.8 us, 32 of 1-2K 42.5 -> 38.6, 16 x 64K 650 ->
-  // 639, one of 32K 30.2 / 30.4 (with a ring of 3: 58.1, 39.5, 640 and 30.8).  The
-  // top-k-list source never does.
+  // 639, one of 32K 30.2 / 30.4 (with a ring of 3: 58.1, 39.5, 640 and 30.8); so does the
+  // top-k-list source (finalize and merge: 16 ragged x 8-64K 46.9 -> 44.4 us, 4 x 30-60K
+  // groups of 8 21.2 -> 20.1, one of 32K 13.7 -> 13.3, 16 x 128K 93.7 -> 93.2).
   constexpr bool kKeyLdsAny =
-      kMfma && kBf16 && D == 128 && ((SRC == kSrcTopkFused && KROWS) || SRC == kSrcLists || SRC == kSrcCondFused || SRC == kSrcDense);
+      kMfma && kBf16 && D == 128 && ((SRC == kSrcTopkFused && KROWS) || SRC == kSrcLists || SRC == kSrcCondFused || SRC == kSrcDense || SRC == kSrcTopk);
   // (the one-launch condition call at G = 8 takes the place of its prologue's statistics,
   // which are dead by then and as large: 145 KiB of LDS instead of 177)
   constexpr bool kKeyOnStats = kKeyLdsAny && SRC == kSrcCondFused && G == 8;
@@ -1349,12 +1350,12 @@ __global__ __launch_bounds__(kFinThreads, 2) void ia_condition_block_paged_final
   // issue: a load issued by consume would make the wave wait for every load in
   // flight (the vector memory counter drains in order).
   auto stream = [&](auto&& issue, auto&& consume) {
-    // The one-launch top-k call's and the dense source's long streams whose consume is the
-    // longer one (keys through LDS, fp8 codes widened) keep one subtile in flight per wave:
-    // a CU then streams faster than with two (C3 -1.0 to -1.2 us, C5 -1.2 us, dense fp8 8
-    // x 4-12K 37.9 -> 36.5 us; same bits).  The condition-rule calls' short streams keep
+    // The long streams whose consume is the longer part of a step (keys through LDS, fp8
+    // codes widened) keep one subtile in flight per wave: a CU then streams faster than
+    // with two (one-launch top-k C3 -1.0 to -1.2 us, C5 -1.2 us, dense fp8 8 x 4-12K 37.9
+    // -> 36.5 us; same bits).  The condition-rule calls' short streams keep
     // the deeper ring for their start.
-    constexpr int NBUF = (SRC == kSrcTopkFused && (KROWS || kFp8)) || (SRC == kSrcDense && (kKeyLdsAny || kFp8)) ? 2 : KV::kRing;
+    constexpr int NBUF = (SRC == kSrcTopkFused && (KROWS || kFp8)) || ((SRC == kSrcDense || SRC == kSrcTopk) && (kKeyLdsAny || kFp8)) ? 2 : KV::kRing;
     // the priority feedback below stays in the fp8 and key-row top-k calls (measured
     // faster with it) and in the finalizes of the multi-launch paths; the uniform bf16
     // top-k call (C4 -0.4, C2 -0.15 us) and the one-launch condition calls (-0.1 to
