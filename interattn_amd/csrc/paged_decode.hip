@@ -276,14 +276,18 @@ int run_topk_decode(const ia_decode_shape* shape, const void* q, const ia_paged_
   p.nb_max = nb_max;
   p.k_per_seq = k_per_seq;
   // Keys as whole rows (through LDS to the operand layout) where a CU streams partly
-  // alone: variable-length batches, and launches whose chosen K/V is under 256 MB, too
-  // little to keep HBM at its rate.  Measured, operand-layout loads against whole rows
-  // (bf16, D = 128; the same results either way): 4 x 30-60K tokens, Quest, 98 blocks of 32
-  // tokens 31.9 / 30.9 us; 8 x 21-85K, 96 of 64 50.3 / 48.3; 6 x 1-4.6K, 104 of 16 22.4 /
-  // 21.3; ten other draws under 256 MB -0.8 to +0.1; one of 32K 17.8 / 17.8.  Above: 16 x
-  // 128K, 64 of 128 (537 MB) 98.0 / 101 (98.5 / 99.7 on another box), 8 x 128K 59.5 / 59.5.
-  const int64_t chosen_bytes = (int64_t)shape->batch * shape->n_kv_heads * k_cap * block_size * D * 4;
-  p.key_rows = k_per_seq != nullptr || chosen_bytes < (1ll << 28);
+  // alone: variable-length batches, and Quest launches (two key rows scored per block:
+  // their items' longer prologues leave the streams out of step) whose waves (256 CUs x 8)
+  // have at least three subtiles each to hide the transpose behind and whose chosen K/V is
+  // under 256 MB, too little to keep HBM at its rate.  Measured, operand-layout loads
+  // against whole rows (bf16, D = 128; the same results either way): Quest 4 x 30-60K, 98
+  // blocks of 32 tokens 31.9 / 30.9 us (read cold 33.5 / 32.6); 8 x 21-85K, 96 of 64 50.3 /
+  // 48.3; 14 x 100K, 14 of 128 44.2 / 43.5.  Mean keys, read cold: 1 x 32K, 67 of 64 18.1 /
+  // 18.6, 4 x 32K 26.6 / 27.0, 8 x 20-40K 37.8 / 38.2; 16 x 128K, 64 of 128 (537 MB) 98.0 /
+  // 101.
+  const int64_t chosen = (int64_t)shape->batch * shape->n_kv_heads * k_cap * (block_size / 16);  // subtiles
+  p.key_rows = k_per_seq != nullptr || (keys->score == IA_SCORE_QUEST && chosen >= 3 * 8 * 256 &&
+                                        chosen * 16 * D * 4 < (1ll << 28));
   p.topk_k = k;
   p.forced_first = forced_first;
   p.forced_last = forced_last;
