@@ -191,7 +191,12 @@ typedef struct ia_block_keys {
  * forced_in_k else k (k_per_seq, a device array [batch], overrides k per sequence
  * when non-NULL).  idx[b, h, 0:n_sel[b,h]] receives the chosen block ids in
  * ascending order (idx row stride k_cap >= k_eff + #forced).  scores may be NULL;
- * otherwise it receives [batch, Hkv, nb_max] float32 (-inf past the end).
+ * otherwise it receives [batch, Hkv, nb_max] float32 (-inf past the end).  Tables
+ * wider than 1024 blocks may run as two launches (scores over the whole device, then
+ * the rule per row: the same results), which need memory for the scores: scores, or
+ * a workspace of ia_select_topk_workspace_size bytes (uninitialised, overwritten).
+ * Tables of up to 8192 blocks run in one launch without either; wider ones need one of
+ * them (IA_ERR_WORKSPACE).
  * The selection rule is the group-mean + torch.topk of CBG/methods/quest.py:91-103;
  * the reference's condition-block path selects by an eps threshold instead
  * (_select_prompt_blocks_triton, CBT/core.py:701-744).

@@ -1,4 +1,6 @@
-// Library-level C ABI: version and per-thread error reporting.
+// Library-level C ABI: version and per-thread error reporting; host queries shared by
+// the launchers.
+#include <atomic>
 #include <string>
 
 #include "ia_common.hpp"
@@ -20,6 +22,18 @@ int check_launch(const char* what) {
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(IA_ERR_LAUNCH, std::string(what) + ": " + hipGetErrorString(e));
   return IA_OK;
+}
+
+int device_cus() {
+  constexpr int kMaxCachedDevices = 64;
+  static std::atomic<int> cached[kMaxCachedDevices];  // (concurrent first calls store the same value)
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 256;
+  if (dev < kMaxCachedDevices) n = cached[dev].load(std::memory_order_relaxed);
+  if (n > 0) return n;
+  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return 256;
+  if (dev < kMaxCachedDevices) cached[dev].store(n, std::memory_order_relaxed);
+  return n;
 }
 
 }  // namespace ia

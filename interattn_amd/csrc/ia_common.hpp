@@ -242,6 +242,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 void set_error(const std::string& msg);
 int fail(int code, const std::string& msg);
 int check_launch(const char* what);
+int device_cus();  // CUs of the current device (256, an MI355X's, where the query fails)
 
 inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 

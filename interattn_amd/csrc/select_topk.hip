@@ -1,8 +1,8 @@
 // Top-k block selection for gfx950: block scorer and per-(sequence, kv head)
 // radix select fused in one launch, one 1024-thread workgroup per (sequence,
-// kv head) (rows of more than 1024 blocks: two launches, below).  A whole score row stays inside one workgroup, so the launch needs
-// no cross-workgroup synchronisation (an agent-scope fence writes back the
-// XCD's L2 and costs far more than the work here).
+// kv head) (wide tables: two launches, below).  A whole score row stays inside
+// one workgroup, so the launch needs no cross-workgroup synchronisation (an
+// agent-scope fence writes back the XCD's L2 and costs far more than the work here).
 //
 //   scoring: score_j = (mean_g q_g) . k_bar_j / sqrt(D); one k_bar row per 16
 //   lanes (4 rows per wave-wide load), 16 (bf16) or 8 (fp32) rows per lane in
@@ -30,7 +30,8 @@ namespace {
 constexpr int kSelThreads = 1024;
 constexpr int kSelWaves = kSelThreads / 64;
 constexpr int kMaxLdsScores = 8192;
-constexpr int kOneLaunchBlocks = 1024;  // rows scored and selected by one workgroup in one launch
+constexpr int kOneLaunchBlocks = 1024;  // tables never selected in two launches (two_launches)
+constexpr int64_t kScoreWgsPerCu = 2;   // scorer workgroups (of 4 waves) per CU, at most
 
 struct SelectParams {
   const void* q;
@@ -48,6 +49,7 @@ struct SelectParams {
   float* scores;  // [batch*Hkv, nb_max] or null
   int32_t n_kv_heads;
   float score_scale;   // 1 / (G * sqrt(D)) (mean key) or 1 / G (Quest)
+  int32_t fill_scores; // the caller reads the scores: -inf past a row's blocks
 };
 
 template <int D, int G, bool QF32, bool KBF16, bool QUEST>
@@ -207,19 +209,32 @@ __global__ __launch_bounds__(kSelThreads) void ia_condition_block_select_topk(Se
 // ---------------------------------------------------------------- long rows: two launches
 //
 // A row of many blocks keeps one workgroup of the kernel above streaming its keys alone
-// (one CU, ~40 GB/s: 99 us for 8 rows of 15,626 bf16 D = 128 blocks, 248 CUs idle).  Long
+// (one CU, ~55 GB/s: 73 us for 8 rows of 15,626 bf16 D = 128 blocks, 248 CUs idle).  Long
 // rows are therefore scored by a launch over the whole device, and a second launch of one
 // workgroup per row selects from the stored scores (the same score arithmetic and rule,
-// so the same bits).  Those 8 rows then take 9 + 11 us: the scorer reads 32 MB at 3.5 TB/s
-// (a workgroup lives for one round trip), and the selection is bound by one CU's vector
-// instructions, about 80 per key over its passes.  Scores held by the threads in registers,
-// strided so that the row is read coalesced: 20.8 us for both launches against 24.1 with
-// the row staged in LDS and 24.7 with 16 consecutive scores per thread (their loads touch
-// 64 lines per instruction).
+// so the same bits).  Those 8 rows then take 17.4 us: the scorer reads 32 MB at ~3.5 TB/s
+// and the selection is bound by one CU's vector instructions, about 80 per key over its
+// passes.  Scores held by the threads in registers, strided so that the row is read
+// coalesced: 20.8 us for both launches (an earlier run) against 24.1 with the row staged in LDS and 24.7
+// with 16 consecutive scores per thread (their loads touch 64 lines per instruction).
+//
+// The table's width is a capacity, its rows are often short (a server sizes tables for the
+// longest context), so both launches work in proportion to each row's own blocks: nothing
+// is stored past them unless the caller asked for the scores, the selection holds as many
+// keys per thread as the row needs, and the scorer's grid is at most kScoreWgsPerCu
+// workgroups per CU, striding over the row (a workgroup that finds its part of the table
+// empty still costs about 2.5 ns of dispatch).  With a grid over the table's width and
+// -inf stored and read back up to it, 1024 rows of 16 / 125 blocks in a 4096-wide table took
+// 84 / 104 us, 256 in a 15,626-wide one 28 / 31; now 9.4 / 15.4 and 6.3 / 8.4.  Grids of 1,
+// 2, 4 and 8 workgroups per CU: 256 rows of 125 blocks 7.8 / 8.4 / 10.3 / 13.5 us, 32 rows of
+// 4096 blocks 13.8 / 12.4 / 12.5 / 12.5, 8 of 15,626 18.4 / 17.6 / 18.3 / 18.2.  (256 full
+// rows of 15,626 are slower than with the whole grid, 193 against 177 us; the next keys'
+// loads issued ahead, and each workgroup on one contiguous part, leave that as it is.)
 
-// Block scores [row, nb_max] (-inf past a row's end): 256 threads score kBlocks
-// consecutive blocks of one row (128 of bf16 D = 128 keys; twice as many per workgroup
-// measured 0.2-1.5 us slower); every key row of a lane is requested before any is used.
+// Block scores [row, nb_max] (with p.fill_scores: -inf past a row's end): 256 threads score
+// kBlocks consecutive blocks of one row (128 of bf16 D = 128 keys; twice as many per workgroup
+// measured 0.2-1.5 us slower), then the next of their stride; every key row of a lane is
+// requested before any is used.
 template <int D, bool KBF16, bool QUEST>
 struct ScoreShape {
   static constexpr int kRowWords = D / 16 * (KBF16 ? 2 : 4) / 4;             // words per lane per key row
@@ -240,14 +255,13 @@ __global__ __launch_bounds__(256) void ia_condition_block_scores(SelectParams p,
   const int r = lane >> 4;
   const int h = blockIdx.y;
   const int b = blockIdx.z;
-  const int base = blockIdx.x * S::kBlocks;
   const int seq_len = max(p.seq_lens[b], 0);
   const int nb = min((seq_len + p.block_size - 1) / p.block_size, p.nb_max);
   float* sc_row = p.scores + ((int64_t)b * p.n_kv_heads + h) * p.nb_max;
-  if (base >= nb) {
-    for (int j = base + threadIdx.x; j < min(base + S::kBlocks, p.nb_max); j += 256) sc_row[j] = kNegInf;
-    return;
-  }
+  if (p.fill_scores)
+    for (int j = nb + (int)(blockIdx.x * 256 + threadIdx.x); j < p.nb_max; j += (int)gridDim.x * 256) sc_row[j] = kNegInf;
+  int base = blockIdx.x * S::kBlocks;
+  if (base >= nb) return;
   // keys: in step t, wave w handles row base + 16 t + 4 w + r (rows past nb re-read row nb - 1)
   const int64_t head = ((int64_t)b * p.kb_batch_stride + (int64_t)h * p.kb_head_stride) * EB;
   const char* kb = reinterpret_cast<const char*>(p.k_bar) + head;
@@ -265,12 +279,15 @@ __global__ __launch_bounds__(256) void ia_condition_block_scores(SelectParams p,
       w[0] = x[0]; w[1] = x[1];
     }
   };
+  auto load_keys = [&]() {
 #pragma unroll
-  for (int t = 0; t < NS; ++t) {
-    const int64_t off = ((int64_t)min(base + 16 * t + 4 * wave + r, nb - 1) * D + c16 * DPL) * EB;
-    load_row(kb + off, w1[t]);
-    if constexpr (QUEST) load_row(kn + off, w2[t]);
-  }
+    for (int t = 0; t < NS; ++t) {
+      const int64_t off = ((int64_t)min(base + 16 * t + 4 * wave + r, nb - 1) * D + c16 * DPL) * EB;
+      load_row(kb + off, w1[t]);
+      if constexpr (QUEST) load_row(kn + off, w2[t]);
+    }
+  };
+  load_keys();
   // mean key: qm = sum_g q_g; Quest: qm = sum_g q_g+, qn = sum_g q_g- (g ascending)
   float qm[DPL], qn[DPL];
 #pragma unroll
@@ -316,31 +333,37 @@ __global__ __launch_bounds__(256) void ia_condition_block_scores(SelectParams p,
       }
     }
   }
-  if constexpr (NS >= 4) {
-    float v[NS];
+  while (true) {
+    if constexpr (NS >= 4) {
+      float v[NS];
 #pragma unroll
-    for (int t = 0; t < NS; ++t)
-      v[t] = QUEST ? block_dot_quest<DPL, KBF16>(w1[t], w2[QUEST ? t : 0], qm, qn) : block_dot<DPL, KBF16>(w1[t], qm);
-    reduce_scatter16<NS>(v, lane);
-    constexpr int kCopies = 16 / NS;  // lanes holding each step
-    const int t = c16 / kCopies;
-    const int j = base + 16 * t + 4 * wave + r;
-    if (c16 % kCopies == 0 && j < p.nb_max) sc_row[j] = j < nb ? v[0] * p.score_scale : kNegInf;
-  } else {
-#pragma unroll
-    for (int t = 0; t < NS; ++t) {
-      const float a = QUEST ? block_score_quest<DPL, KBF16>(w1[t], w2[QUEST ? t : 0], qm, qn, p.score_scale)
-                            : block_score<DPL, KBF16>(w1[t], qm, p.score_scale);
+      for (int t = 0; t < NS; ++t)
+        v[t] = QUEST ? block_dot_quest<DPL, KBF16>(w1[t], w2[QUEST ? t : 0], qm, qn) : block_dot<DPL, KBF16>(w1[t], qm);
+      reduce_scatter16<NS>(v, lane);
+      constexpr int kCopies = 16 / NS;  // lanes holding each step
+      const int t = c16 / kCopies;
       const int j = base + 16 * t + 4 * wave + r;
-      if (c16 == 0 && j < p.nb_max) sc_row[j] = j < nb ? a : kNegInf;
+      if (c16 % kCopies == 0 && j < nb) sc_row[j] = v[0] * p.score_scale;
+    } else {
+#pragma unroll
+      for (int t = 0; t < NS; ++t) {
+        const float a = QUEST ? block_score_quest<DPL, KBF16>(w1[t], w2[QUEST ? t : 0], qm, qn, p.score_scale)
+                              : block_score<DPL, KBF16>(w1[t], qm, p.score_scale);
+        const int j = base + 16 * t + 4 * wave + r;
+        if (c16 == 0 && j < nb) sc_row[j] = a;
+      }
     }
+    base += (int)gridDim.x * S::kBlocks;
+    if (base >= nb) return;
+    load_keys();
   }
 }
 
 // The rule on a stored score row, one workgroup per row: thread t holds the keys of
-// blocks t + 1024 e, e < KPT, in registers (KPT = 0: rows longer than 32 keys per thread are
-// read from memory in every pass).
-template <int KPT>
+// blocks t + 1024 e, e < K, in registers, K the least of 1, 4, 8, 16 and 32 that covers
+// the row's own blocks (a row longer than 32 keys per thread is read from memory in every
+// pass).  KMAX: the K of the table's width, 0 where 32 does not cover it.
+template <int KMAX>
 __global__ __launch_bounds__(kSelThreads) void ia_condition_block_select_scores(SelectParams p) {
   __shared__ TopkLds<kSelThreads> sel_lds;
   const int h = blockIdx.x;
@@ -353,15 +376,27 @@ __global__ __launch_bounds__(kSelThreads) void ia_condition_block_select_scores(
   const TopkRule rule{p.forced_first, p.forced_last, k_b, p.forced_in_k, p.k_cap};
   int32_t* out_idx = p.idx + (int64_t)bh * p.k_cap;
   auto emit = [&](int pos, int j) { out_idx[pos] = j; };
-  int n;
-  if constexpr (KPT > 0) {
-    u32 key[KPT];
+  int n = 0;
+  auto held = [&](auto kc) {
+    constexpr int K = decltype(kc)::value;
+    u32 key[K];
 #pragma unroll
-    for (int e = 0; e < KPT; ++e)  // (entries past the row's blocks hold -inf; past nb_max: unused)
-      key[e] = order_key(sc_row[min((int)threadIdx.x + kSelThreads * e, p.nb_max - 1)]);
-    n = topk_select_regs<kSelThreads, KPT>(sel_lds, key, nb, rule, emit);
-  } else {
-    n = topk_select<kSelThreads>(sel_lds, [&](int j) -> u32 { return order_key(sc_row[j]); }, nb, rule, emit);
+    for (int e = 0; e < K; ++e)  // (entries past the row's blocks: unused)
+      key[e] = order_key(sc_row[max(min((int)threadIdx.x + kSelThreads * e, nb - 1), 0)]);
+    n = topk_select_regs<kSelThreads, K>(sel_lds, key, nb, rule, emit);
+  };
+  constexpr int kTop = KMAX == 0 ? 32 : KMAX;
+  if (nb <= kSelThreads) held(std::integral_constant<int, 1>{});
+  else if (kTop == 4 || nb <= 4 * kSelThreads) held(std::integral_constant<int, 4>{});
+  else if constexpr (kTop >= 8) {
+    if (kTop == 8 || nb <= 8 * kSelThreads) held(std::integral_constant<int, 8>{});
+    else if constexpr (kTop >= 16) {
+      if (kTop == 16 || nb <= 16 * kSelThreads) held(std::integral_constant<int, 16>{});
+      else if constexpr (kTop >= 32) {
+        if (KMAX == 32 || nb <= 32 * kSelThreads) held(std::integral_constant<int, 32>{});
+        else n = topk_select<kSelThreads>(sel_lds, [&](int j) -> u32 { return order_key(sc_row[j]); }, nb, rule, emit);
+      }
+    }
   }
   if (threadIdx.x == 0) p.n_sel[bh] = n;
 }
@@ -369,11 +404,39 @@ __global__ __launch_bounds__(kSelThreads) void ia_condition_block_select_scores(
 template <int D, bool KBF16, bool QUEST>
 void launch_scores(const SelectParams& p, int group, bool qf32, int batch, hipStream_t st) {
   constexpr int kBlocks = ScoreShape<D, KBF16, QUEST>::kBlocks;
-  const dim3 grid((p.nb_max + kBlocks - 1) / kBlocks, p.n_kv_heads, batch);
+  const int64_t rows = (int64_t)p.n_kv_heads * batch;
+  const int64_t per_row = std::max<int64_t>(1, (kScoreWgsPerCu * device_cus() + rows - 1) / rows);
+  const dim3 grid((unsigned)std::min<int64_t>((p.nb_max + kBlocks - 1) / kBlocks, per_row), p.n_kv_heads, batch);
   // the query rows as vector loads where every row starts 16-byte aligned
   const int64_t es = qf32 ? 4 : 2;
   const int q_vec = reinterpret_cast<uintptr_t>(p.q) % 16 == 0 && p.q_batch_stride * es % 16 == 0 && p.q_row_stride * es % 16 == 0;
   hipLaunchKernelGGL((ia_condition_block_scores<D, KBF16, QUEST>), grid, dim3(256), 0, st, p, group, qf32 ? 1 : 0, q_vec);
+}
+
+// Whether a table of nb_max blocks and `rows` rows is selected in two launches (given
+// memory for the scores; wider than kMaxLdsScores there is no other way).  The host knows
+// the capacity, not the rows' lengths, so the line weighs the launch boundary that a short
+// row pays (1.2 - 1.9 us) against what a long row gains.  Graph replays, bf16 D = 128, one
+// launch / two, row lengths 125, 1000 and the table's:
+//     8 rows, 2048-wide    6.0 / 7.3    9.0 / 7.9   12.4 / 9.1
+//    32 rows, 4096-wide    6.3 / 7.7    9.2 / 8.4   26.2 / 13.1
+//    64 rows, 2048-wide    6.4 / 8.1    9.3 / 8.9   17.0 / 13.1
+//   128 rows, 4096-wide    6.4 / 8.0   11.6 / 11.8  31.0 / 28.1
+//   128 rows, 8192-wide    6.4 / 8.0   11.5 / 11.4  55.6 / 50.7
+//   256 rows, 4096-wide    6.6 / 8.3   15.3 / 16.2  48.8 / 48.7
+//   512 rows, 4096-wide   11.4 / 9.5   31.1 / 26.3  97.9 / 93.3
+//  1024 rows, 4096-wide   22.0 / 15.3  61.5 / 50.9   191 / 194
+//  1024 rows, 8192-wide   21.9 / 18.6  57.7 / 54.5   342 / 398
+// Few rows leave the CUs idle in one launch, and the gain is large.  The more rows there
+// are, the wider the table has to be: kMaxLdsScores blocks at one row per CU, in proportion
+// below.  From two rows per CU on the one-launch workgroups (1024 threads of up to 123
+// registers, one per CU) run in rounds, and two launches are faster but for full rows; past
+// 4096 blocks the second launch, which the scorer does not overlap, costs those too much.
+bool two_launches(int nb_max, int64_t rows) {
+  if (nb_max > kMaxLdsScores) return true;
+  const int64_t cus = device_cus();
+  if (rows >= 2 * cus) return nb_max > kOneLaunchBlocks && nb_max <= kMaxLdsScores / 2;
+  return nb_max > std::max<int64_t>(kOneLaunchBlocks, kMaxLdsScores * rows / cus);
 }
 
 // p.scores set: score over the whole device, then select per row
@@ -541,15 +604,10 @@ int ia_select_topk(const ia_decode_shape* shape, const void* q, const ia_block_k
   p.scores = scores;
   p.n_kv_heads = shape->n_kv_heads;
   p.score_scale = score_scale;
-  // Long rows in two launches, given memory for their scores.  The line: one workgroup
-  // streams its row's keys alone, and from the second key batch on (above 1024 blocks of
-  // bf16 D = 128) that costs more than a second launch.  One launch against two (graph
-  // replays, 8 kv heads): 8 rows of 1024 blocks 9.3 / 8.7 us, 2048 16.2 / 9.7, 4096 26.2 /
-  // 10.3, 15626 100.5 / 20.8, 32768 201 / 35.5; 128 rows of 1024 blocks 13.3 / 14.0, 2048
-  // 21.6 / 19.3, 4096 32.7 / 29.4.
   float* stored = scores ? scores : (workspace && workspace_bytes >= need ? reinterpret_cast<float*>(workspace) : nullptr);
-  if (stored && nb_max > kOneLaunchBlocks) {
+  if (stored && two_launches(nb_max, (int64_t)shape->batch * shape->n_kv_heads)) {
     p.scores = stored;
+    p.fill_scores = scores != nullptr;
     return run_two_launches(p, D, G, shape->q_dtype == IA_F32, keys->dtype == IA_BF16, shape->batch,
                             reinterpret_cast<hipStream_t>(stream));
   }

@@ -477,7 +477,7 @@ __device__ __forceinline__ int topk_select(TopkLds<NT>& L, KeyAt key_at, int nb,
 // Places in block order for topk_select_regs: bit e of a thread's bits marks block t + NT e.
 // pre[e * waves + w] receives the marked blocks before wave w's part of stripe e (a scan
 // of the stripes' wave counts in block order); returns all marked blocks.  Every thread
-// calls it; two barriers.
+// calls it; three barriers.
 template <int NT, int KPT>
 __device__ __forceinline__ int stripe_prefix(u32 bits, int* pre) {
   constexpr int kWv = NT / 64;
