@@ -1,7 +1,9 @@
 """The one-launch eps-rule and fixed-mask calls with GQA groups of 8: against the
-multi-launch path on the same inputs (selection equal away from eps, outputs within the
-rounding of two orders of the same sums), at the edges of an item's blocks; the hand-off
-fallback bit for bit; what does not fit stays on the multi-launch path."""
+multi-launch path on the same inputs (the same selection, eps in a gap of the conditions;
+outputs within the rounding of two splits of the same sums, in proportion to the outputs),
+at the edges of an item's blocks; the hand-off fallback bit for bit; what does not fit stays
+on the multi-launch path; the entry points for groups of up to 4 equal this one and refuse
+groups of 8."""
 
 import numpy as np
 import pytest
@@ -10,6 +12,7 @@ import torch
 from interattn_amd import _native as N
 from interattn_amd import condition_block as cb
 from tests._util import announce
+from tests.test_gpu_condition import _np, _oracle_stats, _prefix_np
 
 pytestmark = pytest.mark.gpu
 
@@ -48,18 +51,34 @@ def _fused(ws):
 
 
 def _eps(x):
-    """An eps in the widest gap of the conditions' upper half (so both orders of the sums
-    select the same blocks), from the standalone selection by bisection."""
-    lo, hi = -9.0, 3.0
-    nb = x["prefix"]["block_valid_counts"].numel()
-    for _ in range(30):
-        mid = 0.5 * (lo + hi)
-        share = float(cb._select_prompt_blocks_triton(x["q"], x["prefix"], 10.0 ** mid)[0].float().mean())
-        if share > (0.05 if nb > 40 else 0.5):
-            lo = mid
-        else:
-            hi = mid
-    return 10.0 ** hi
+    """An eps that selects about 5% of the blocks (half of a few), in the middle of the
+    widest relative gap there between the conditions' 64-bit values.  Float32 logits of up to
+    ~20 leave a condition ~1e-5 of relative rounding, so either order of the row's sums
+    selects the same blocks."""
+    q = _np(x["q"].float())[:, :, 0]
+    mean = _oracle_stats(q.reshape(-1, q.shape[-1]), _prefix_np(x["prefix"]), 8, False)[1]
+    v = np.sort(mean[mean > 0])[::-1]
+    n = (0.05 if x["prefix"]["block_valid_counts"].numel() > 40 else 0.5) * len(v)
+    lo = max(int(0.5 * n), 1)
+    hi = min(max(int(1.5 * n), lo + 1), len(v) - 1)
+    i = lo + int(np.argmax(v[lo - 1:hi - 1] / v[lo:hi])) if hi > lo else lo
+    assert v[i - 1] / v[i] > 1.0002, "no gap wide enough"
+    return float(np.sqrt(v[i - 1] * v[i]))
+
+
+def _check(got, ref, dt):
+    """Two splits of the same sums.  bf16 caches: every softmax weight is rounded to bf16
+    against its item's own maximum, a relative error of at most 2^-9 and ~0.42 x 2^-9 rms, so
+    independent roundings on both sides leave ~0.42 sqrt(2) 2^-9 = 1.2e-3 of the output's
+    2-norm whatever cancels in the sum; float32 caches keep float32 sums (a few 1e-7).  Bounds:
+    ~3.5 of those rms, and 4 times that on single values (13 sigma).  An item's partial that is
+    lost or counted twice moves the output by ~1 / sqrt(items) > 0.1."""
+    got, ref = _np(got).astype(np.float64), _np(ref).astype(np.float64)
+    rel = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    rms = np.sqrt(np.mean(ref ** 2))
+    bound = 2.0 ** -8 if dt == "bf16" else 2e-6
+    assert rel <= bound, (rel, bound)
+    assert np.abs(got - ref).max() <= 4 * bound * rms, (np.abs(got - ref).max() / rms, bound)
 
 
 @pytest.mark.parametrize("c", CASES, ids=[f"h{c[0]}d{c[1]}b{c[2]}p{c[3]}_{c[5]}" for c in CASES])
@@ -67,7 +86,6 @@ def test_one_launch_equals_multi_launch(c, device, monkeypatch):
     hkv, d, block, p, s, dt, mixed, kbd = c
     announce(f"group of 8: {c}")
     x = _inputs(c, device)
-    tol = 2e-2 if dt == "bf16" else 1e-4
     for eps in (0.0, _eps(x), 1e30):
         got = {}
         for one in ("1", "0"):
@@ -75,10 +93,9 @@ def test_one_launch_equals_multi_launch(c, device, monkeypatch):
             ws = {}
             got[one] = _call(x, block, p, eps, ws)
             assert _fused(ws) == (one == "1")
-        differ = int((got["1"][1] != got["0"][1]).sum())
-        assert differ == 0 or (0.0 < eps < 1e30 and differ <= 8), (eps, differ)  # one block at eps: its 8 rows
-        if differ == 0:
-            np.testing.assert_allclose(got["1"][0].cpu().numpy(), got["0"][0].cpu().numpy(), atol=tol, rtol=0)
+        assert torch.equal(got["1"][1], got["0"][1]), eps
+        assert bool(got["0"][1].any()) == (eps < 1e30)
+        _check(got["1"][0], got["0"][0], dt)
     mask = torch.zeros((hkv, x["prefix"]["block_valid_counts"].numel()), device=device, dtype=torch.bool)
     mask[:, ::5] = True
     out = []
@@ -86,8 +103,8 @@ def test_one_launch_equals_multi_launch(c, device, monkeypatch):
         monkeypatch.setenv("INTERATTN_CONDITION_ONE_LAUNCH", one)
         out.append(cb.fixed_mask_hybrid_attention(
             q_grouped=x["q"], prompt_prefix=x["prefix"], selected=mask, k_suffix=x["ks"], v_suffix=x["vs"],
-            block_size=block, output_dtype=torch.float32, workspace={}).cpu().numpy())
-    np.testing.assert_allclose(out[0], out[1], atol=tol, rtol=0)
+            block_size=block, output_dtype=torch.float32, workspace={}))
+    _check(out[0], out[1], dt)
 
 
 def test_handoff_fallback_and_replays_are_exact(device, monkeypatch):
@@ -113,3 +130,46 @@ def test_fp32_head_dim_128_keeps_the_multi_launch_path(device, monkeypatch):
     ws = {}
     _call(x, 64, 3000, 0.01, ws)
     assert not _fused(ws)
+
+
+@pytest.mark.parametrize("group", [1, 2, 4, 8])
+def test_entry_points_for_groups_of_up_to_four(group, device):
+    """``ia_condition_decode_fused`` and ``ia_fixed_mask_decode_fused`` through the C ABI: the
+    bits of ``ia_condition_one_launch`` for groups of up to 4, a refusal for groups of 8."""
+    announce(f"one-launch entry points, group of {group}")
+    hkv, d, block, p, s = 2, 128, 64, 5000, 9
+    x = _inputs((hkv, d, block, p, s, "bf16", True, "bf16"), device)
+    q, sh = cb._grouped_shape(x["q"][:, :group].contiguous())
+    sm, keep, nb = cb._summaries_desc(x["prefix"], hkv, d)
+    kv = cb._kv_desc(x["prefix"]["k_block_attn"], x["prefix"]["v_block_attn"], block)
+    sfx, keep_s = cb._suffix_desc(x["ks"], x["vs"], x["len"], torch.bfloat16)
+    lib = N.lib()
+    n = lib.ia_condition_decode_fused_workspace_size(1, hkv, group, d)
+    stream = torch.cuda.current_stream().cuda_stream
+    mask = torch.zeros((hkv, nb), device=device, dtype=torch.uint8)
+    mask[:, ::7] = 1
+    eps, scale = 0.02, d ** -0.5
+
+    def run(call):
+        out = torch.empty((hkv * group, d), device=device, dtype=torch.float32)
+        sel = torch.zeros((hkv * group, nb), device=device, dtype=torch.uint8)
+        ws = torch.zeros((n,), device=device, dtype=torch.uint8)
+        rc = call(out.data_ptr(), sel.data_ptr(), ws.data_ptr())
+        torch.cuda.synchronize()
+        return rc, out, sel
+
+    new = [run(lambda o, sl, w, m=m: lib.ia_condition_one_launch(
+        sh, q.data_ptr(), sm, m, kv, sfx, eps, 0, sl, scale, o, N.IA_F32, w, n, stream)) for m in (None, mask.data_ptr())]
+    old = [run(lambda o, sl, w: lib.ia_condition_decode_fused(sh, q.data_ptr(), sm, kv, sfx, eps, 0, sl, scale, o,
+                                                              N.IA_F32, w, n, stream)),
+           run(lambda o, sl, w: lib.ia_fixed_mask_decode_fused(sh, q.data_ptr(), sm, mask.data_ptr(), kv, sfx, scale, o,
+                                                               N.IA_F32, w, n, stream))]
+    assert lib.ia_condition_one_launch_items(sh, sm, N.IA_BF16, sfx.cap) > 0 and all(r[0] == N.IA_OK for r in new)
+    assert (lib.ia_condition_decode_fused_items(sh, sm, N.IA_BF16, sfx.cap) > 0) == (group <= 4)
+    for a, b in zip(old, new):
+        if group > 4:
+            assert a[0] == N.IA_ERR_UNSUPPORTED
+        else:
+            assert a[0] == N.IA_OK and torch.equal(a[1], b[1]) and torch.equal(a[2], b[2])
+    assert bool(new[0][2].any()) and not bool(new[1][2].any())  # (a mask's call writes no selection)
+    del keep, keep_s
