@@ -421,7 +421,7 @@ IA_API int ia_fixed_mask_decode(const ia_decode_shape* shape, const void* q,
  * the waiting item itself, so the result never depends on timing.  (When every row
  * has the same work and a row has at most two items, each item scores the whole
  * row itself instead, with the same arithmetic.  Launches with k_per_seq (the
- * variable-length batches) and Quest launches of about 50 to 256 MB of chosen K/V load
+ * variable-length batches) and Quest launches of at least 2.5 chosen subtiles of 16 tokens per resident wave load
  * the keys as whole rows and pass them through LDS to the matrix-core operand layout, which
  * streams faster where HBM is not kept at its rate; the words reaching the products are
  * the same.)  Equal to

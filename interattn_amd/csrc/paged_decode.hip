@@ -232,6 +232,30 @@ FusedWs fused_ws_layout(int batch, int hkv, int g, int d, int nb_max, int k_cap,
   return L;
 }
 
+// Keys as whole rows (through LDS to the operand layout) where a CU streams partly alone:
+// variable-length batches (k_per_seq), and Quest launches (two key rows scored per block)
+// of at least 2.5 chosen subtiles per wave (8 waves per CU): the whole-row instance keeps
+// one subtile in flight per wave, the operand-layout one two, so a wave with two has both
+// in flight from the start only there.  Measured, operand-layout loads against whole rows
+// (bf16, D = 128, us; the same results either way), by subtiles per wave:
+//                                             2.0          2.25          2.5           3           16           48
+//   8 x 21-85K, blocks of 64             24.2 / 24.2  25.0 / 24.7  25.8 / 25.3  27.3 / 26.3  60.0 / 60.0
+//   4 x 30-60K, G = 8, blocks of 32      26.5 / 27.0  27.4 / 27.5  28.4 / 28.2  29.8 / 29.2  61.8 / 61.2
+//   1 x 32K, blocks of 64                20.0 / 20.5               21.5 / 21.4  23.1 / 22.2
+//   8 x 60-120K, G = 8, blocks of 64                                                         68.2 / 67.3  146 / 144
+//   16 x 100K, blocks of 128                                                                 63.3 / 63.1  144 / 143
+// At 1.5 and less whole rows measured 0 - 2% faster again (not taken: one line).  Mean keys,
+// read cold, have the operand layout faster: 1 x 32K, 67 blocks of 64 18.1 / 18.6, 4 x 32K 26.6 / 27.0, 8 x 20-40K 37.8 / 38.2;
+// 16 x 128K, 64 of 128 98.0 / 101.
+bool quest_key_rows(int score, int64_t rows, int nb_max, int block_size, int k, int forced_first, int forced_last,
+                    int forced_in_k, int k_cap) {
+  if (score != IA_SCORE_QUEST) return false;
+  // the most blocks a row can choose (k_cap is a capacity)
+  const int64_t forced = (int64_t)forced_first + forced_last;
+  const int64_t most = std::min<int64_t>({k_cap, nb_max, forced_in_k ? std::max<int64_t>(k, forced) : k + forced});
+  return 2 * rows * most * (block_size / 16) >= 5 * 8 * (int64_t)device_cus();
+}
+
 int run_topk_decode(const ia_decode_shape* shape, const void* q, const ia_paged_kv* kv, const int32_t* seq_lens,
                     const ia_block_keys* keys, int32_t block_size, int32_t nb_max, int32_t k,
                     const int32_t* k_per_seq, int32_t forced_first, int32_t forced_last, int32_t forced_in_k,
@@ -275,19 +299,9 @@ int run_topk_decode(const ia_decode_shape* shape, const void* q, const ia_paged_
   p.unit_tokens = block_size;
   p.nb_max = nb_max;
   p.k_per_seq = k_per_seq;
-  // Keys as whole rows (through LDS to the operand layout) where a CU streams partly
-  // alone: variable-length batches, and Quest launches (two key rows scored per block:
-  // their items' longer prologues leave the streams out of step) whose waves (256 CUs x 8)
-  // have at least three subtiles each to hide the transpose behind and whose chosen K/V is
-  // under 256 MB, too little to keep HBM at its rate.  Measured, operand-layout loads
-  // against whole rows (bf16, D = 128; the same results either way): Quest 4 x 30-60K, 98
-  // blocks of 32 tokens 31.9 / 30.9 us (read cold 33.5 / 32.6); 8 x 21-85K, 96 of 64 50.3 /
-  // 48.3; 14 x 100K, 14 of 128 44.2 / 43.5.  Mean keys, read cold: 1 x 32K, 67 of 64 18.1 /
-  // 18.6, 4 x 32K 26.6 / 27.0, 8 x 20-40K 37.8 / 38.2; 16 x 128K, 64 of 128 (537 MB) 98.0 /
-  // 101.
-  const int64_t chosen = (int64_t)shape->batch * shape->n_kv_heads * k_cap * (block_size / 16);  // subtiles
-  p.key_rows = k_per_seq != nullptr || (keys->score == IA_SCORE_QUEST && chosen >= 3 * 8 * 256 &&
-                                        chosen * 16 * D * 4 < (1ll << 28));
+  p.key_rows = k_per_seq != nullptr ||
+               quest_key_rows(keys->score, (int64_t)shape->batch * shape->n_kv_heads, nb_max, block_size, k,
+                              forced_first, forced_last, forced_in_k, k_cap);
   p.topk_k = k;
   p.forced_first = forced_first;
   p.forced_last = forced_last;

@@ -423,10 +423,11 @@ def test_fused_topk_decode_k_per_seq_and_fallback(device):
 ], ids=["g4_p16", "g8_p32", "g2_p16", "g1_p64"])
 def test_key_row_instance_equals_two_step(hq, hkv, page, lens, device):
     """Launches with per-sequence k at head_dim 128 run the instance that loads keys as
-    whole rows and passes them through LDS to the MFMA operand layout; the words that
-    reach the products are the ones the operand-layout loads give, so the output equals
-    the two-step path bit for bit, for every group size, page size and ragged length
-    (one-token sequences and partial subtiles included)."""
+    whole rows and passes them through LDS to the MFMA operand layout; its output equals
+    the two-step path's bit for bit, for every group size, page size and ragged length
+    (one-token sequences and partial subtiles included).  The two-step finalize loads keys
+    the same way: tests/test_gpu_key_loads.py compares both with the operand-layout loads,
+    which give the products the same words."""
     announce(f"key-row instance: G={hq // hkv} page={page} lens={lens}")
     case = make_case(seed=31 + page + hq, batch=len(lens), hq=hq, hkv=hkv, d=128, seq_lens=lens, page_size=page)
     dev = to_dev(case, device)
