@@ -33,10 +33,16 @@ def _code(dtype, what):
         raise ValueError(f"{what}: unsupported dtype {dtype}") from None
 
 
+# torch's own accessor of the raw handle: it builds no ``torch.cuda.Stream`` object (2 us of a
+# call's 19 us on the host).  It is not public API, so a torch without it takes the public one.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(t):
-    """The raw handle of torch's current stream on ``t``'s device (without building a
-    ``torch.cuda.Stream`` object, which took 2 us of a call's 19 us on the host)."""
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    """The raw handle of torch's current stream on ``t``'s device."""
+    if _raw_stream is None:
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.get_device())
 
 
 def _require_cuda(*tensors):
