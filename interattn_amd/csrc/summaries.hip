@@ -1,9 +1,9 @@
 // Per-block summaries of a paged K/V pool for gfx950 (the paged form of
 // _build_prompt_blocks, CBT/core.py:449-500).
 //
-//   grid = (blocks, Hkv, batch), 256 threads; a block's keys are summarised by one wave
-//   and its values by another (four blocks a workgroup where only the mean keys are
-//   asked for, else two; more in large launches).  Tokens are read 16 at a time (one
+//   grid = (block groups x Hkv, batch), the kv head fastest, 256 threads; a block's keys
+//   are summarised by one wave and its values by another (four blocks a workgroup where
+//   only the mean keys are asked for, else two; more in large launches).  Tokens are read 16 at a time (one
 //   page-resident subtile), 4 token rows per wave-wide load, 16 lanes per row
 //   (DPL = D/16 dims per lane).  Sums are fp32 (the reference's
 //   dtype=torch.float32 accumulation), extrema are exact copies, and the value
@@ -19,8 +19,8 @@
 //     blocks: the next three subtiles' rows load while one is summed;
 //   * K and V are read by different waves (their sums, extrema and norms together left
 //     room for one subtile in flight per wave at half the waves), and V is not read
-//     unless v_bar, its norms or the extrema are asked for: a top-k program keeps only
-//     the mean keys;
+//     unless v_bar or its norms are asked for: a top-k program keeps only the mean keys
+//     (with the extrema alone the values' waves are launched and leave at once);
 //   * a block's rows are stored as 16-byte pieces, one array per lane row.
 //   Measured (8 sequences of 40-64K tokens, 8 kv heads, D = 128, 64-token blocks, 16-token
 //   pages; before -> after): bf16, every output 381 -> 319 us (5.3 TB/s of the bytes read
@@ -403,14 +403,16 @@ int run_summaries(const ia_paged_kv* kv, const int32_t* old_seq_lens, const int3
   const bool all = v_bar || k_max || k_min || v_norm_max;
   p.window_blocks = window_blocks;
   // Consecutive blocks per wave: enough that a wave's ring runs over about 16 subtiles
-  // (8 where V is not read) instead of draining at every block, as long as the launch
-  // keeps four rounds of resident waves (256 CUs x 12).  Measured, 8 x 40-64K tokens of
+  // (8 where only the mean keys are asked for) instead of draining at every block, as long
+  // as the launch keeps 48 waves per CU: four rounds of the D = 128 instances with every
+  // output (12 resident waves per CU), three of the mean keys' (16), fewer of the D = 64
+  // ones (16 to 32).  Measured, 8 x 40-64K tokens of
   // bf16 D = 128, every output: 64-token blocks 343 us with one block per wave, 326 / 319
   // / 326 us with 8 / 16 / 32 subtiles; 16-token blocks 721 -> 422 us; mean keys only,
   // 144 / 144 / 146 / 151 us with 4 / 8 / 16 / 32.  A batch of 2 x 30K: 49.7 us with one
   // block per wave, 51.6 with two.
   const int64_t waves = (int64_t)window_blocks * n_kv_heads * batch * (all ? 2 : 1);
-  p.wave_blocks = (int)std::max<int64_t>(1, std::min<int64_t>((all ? 16 : 8) / (block_size / 16), waves / 12288));
+  p.wave_blocks = (int)std::max<int64_t>(1, std::min<int64_t>((all ? 16 : 8) / (block_size / 16), waves / (48 * device_cus())));
   const int per_wg = (all ? 2 : 4) * p.wave_blocks;  // blocks per workgroup
   dim3 grid((window_blocks + per_wg - 1) / per_wg * n_kv_heads, batch);
   if (head_dim == 128) all ? launch_summaries<128, true>(p, eb, grid, st) : launch_summaries<128, false>(p, eb, grid, st);
