@@ -168,3 +168,26 @@ def test_line_between_one_launch_and_two(b, hkv, nb_max, device):
             m = int(nbs[i])
             sel = S.select_topk(ref[2][i, 0].cpu().numpy(), m, 30, 2, 1, False)
             assert np.array_equal(got[0][i, 0, :int(got[1][i, 0])].cpu().numpy(), sel)
+
+
+def test_captured_call_follows_the_lengths(device):
+    """A captured selection from a wide table, replayed while its rows grow, shrink and empty."""
+    announce("wide table: captured call")
+    gen = torch.Generator(device=device)
+    gen.manual_seed(3)
+    b, nb_max, block = 2, 5000, 16
+    kb = torch.randn((b, HKV, nb_max, D), device=device, generator=gen).bfloat16()
+    q = torch.randn((b, 4 * HKV, D), device=device, generator=gen).bfloat16()
+    seq = torch.zeros((b,), device=device, dtype=torch.int32)
+    kw = dict(block_size=block, forced_first=1, forced_last=2)
+    ws = {}
+    ia.select_blocks_topk(q, kb, seq, 40, workspace=ws, **kw)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = ia.select_blocks_topk(q, kb, seq, 40, workspace=ws, **kw)
+    for lens in ((300, 80000), (80000, 17000), (0, 16), (65537, 16385)):
+        seq.copy_(torch.tensor(lens, dtype=torch.int32))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert _same(ia.select_blocks_topk(q, kb, seq, 40, **kw), got), lens
