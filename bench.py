@@ -735,8 +735,8 @@ def run_condition(args, w, dev, with_dense, with_cpu, name=None):
         for L in layers:
             call(L)
     torch.cuda.synchronize()
-    # the condition-rule call is four launches (statistics, route, finalize, merge): it
-    # is timed as hipGraph replays, as the reference decodes (stream launches from
+    # the condition-rule call (one launch where it fits, else statistics, route, finalize and
+    # merge) is timed as hipGraph replays, as the reference decodes (stream launches from
     # Python would time the host)
     use_graph = True
     if use_graph:
@@ -878,7 +878,7 @@ def run_condition(args, w, dev, with_dense, with_cpu, name=None):
         "algorithmic_bytes": {"total": total, "q_out": qo_b, "summaries": summ_b, "representatives": rep_b,
                               "selected_kv_and_suffix": kv_b},
         "roofline": {"bound": "hbm",
-                     "kernel": ("ia_condition_decode_fused (one launch: statistics, hand-off, routing, "
+                     "kernel": ("ia_condition_one_launch (one launch: statistics, hand-off, routing, "
                                 "representatives, selected pages, merge)") if eps_one else
                                "statistics, route, finalize and merge launches",
                      "achieved": round(gbps, 1), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
@@ -896,7 +896,7 @@ def run_condition(args, w, dev, with_dense, with_cpu, name=None):
                        "vs_published": round(fixed_us / w["published_fixed_us"], 4),
                        "note": "fixed_mask_hybrid_attention with this call's selection as the mask (the "
                                "reference's 'fixed real mask' run): " +
-                               ("one launch, ia_fixed_mask_decode_fused" if fixed_one else
+                               ("one launch, ia_condition_one_launch" if fixed_one else
                                 "route, finalize and merge launches"),
                        "traffic": traffic_of(f"{name}_fixed")[0] if name and fixed_one else None},
         "cpu_baseline": cpu,

@@ -382,10 +382,14 @@ IA_API int ia_fixed_mask_decode_fused(const ia_decode_shape* shape, const void* 
 /*
  * ia_condition_decode_fused and (mask non-NULL: eps, term1_mass_exp and selected are
  * not read) ia_fixed_mask_decode_fused for every GQA group they have an instance for:
- * groups of 1, 2 and 4 as those two, and of 8 on bf16 caches or at head_dim 64.  The
- * same workspace, semantics and results; ia_condition_one_launch_items is the fit
- * query, 0 when the call does not fit one launch.  Replaces the same reference
- * functions.
+ * groups of 1, 2 and 4, where it is the same launch with the same bits (those two stay
+ * for callers that have them), and of 8 on bf16 caches or at head_dim 64, which those two
+ * refuse.  The same workspace and rule; against ia_condition_decode and
+ * ia_fixed_mask_decode the sums are taken in another split, so softmax weights round to
+ * bf16 against other maxima (bf16 caches: outputs of both differ by up to about 1e-3 of
+ * their 2-norm, with the same error against exact arithmetic).
+ * ia_condition_one_launch_items is the fit query, 0 when the call does not fit one
+ * launch.  Replaces the same reference functions.
  */
 IA_API int32_t ia_condition_one_launch_items(const ia_decode_shape* shape, const ia_block_summaries* sm,
                                              int32_t kv_dtype, int32_t suffix_cap);
@@ -478,8 +482,8 @@ IA_API int ia_sparse_topk_decode_noalloc(const ia_decode_shape* shape, const voi
 
 /*
  * Bound of every wait of one workgroup on another inside the one-launch calls
- * (ia_sparse_topk_decode and its no-alloc form, ia_condition_decode_fused,
- * ia_fixed_mask_decode_fused), in ticks of the GPU's 100 MHz constant clock
+ * (ia_sparse_topk_decode and its no-alloc form, ia_condition_one_launch,
+ * ia_condition_decode_fused, ia_fixed_mask_decode_fused), in ticks of the GPU's 100 MHz constant clock
  * (default 20,000 = 200 us, ~15x the longest prologue; a negative value restores
  * it).  Returns the previous bound.  Applies to calls issued after it on any
  * thread.  A wait that reaches the bound makes the waiting item compute the missing

@@ -306,8 +306,9 @@ def _suffix_desc(k_suffix, v_suffix, suffix_len_dev, prompt_dtype):
 
 def _one_launch():
     """The condition rule's decode and the fixed-mask decode run as one launch
-    (``ia_condition_one_launch``) where the call fits one, unless ``INTERATTN_CONDITION_ONE_LAUNCH=0`` asks for the multi-launch paths
-    (statistics, route, finalize, merge; route, finalize, merge)."""
+    (``ia_condition_one_launch``) where the call fits one, unless
+    ``INTERATTN_CONDITION_ONE_LAUNCH=0`` asks for the multi-launch paths (statistics, route,
+    finalize, merge; route, finalize, merge)."""
     return os.environ.get("INTERATTN_CONDITION_ONE_LAUNCH", "1") != "0"
 
 

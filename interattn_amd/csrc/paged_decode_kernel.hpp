@@ -778,7 +778,8 @@ __global__ __launch_bounds__(kFinThreads, 2) void ia_condition_block_paged_final
   // condition calls' few-subtile items).  Where every workgroup streams equal shares
   // at the HBM rate the transpose costs more than it gains (C4 +0.66 us), so the
   // one-launch top-k call takes it in its KROWS instance only (the host picks that
-  // one for launches with per-sequence k, its variable-length batches).  The dense source
+  // one for launches with per-sequence k, its variable-length batches, and for the larger
+  // Quest launches: quest_key_rows).  The dense source
   // takes it with a ring of 2 (its consume is then the longer part of a step): 8 ragged
   // sequences of 4-12K tokens 60.6 -> 56.8 us, 32 of 1-2K 42.5 -> 38.6, 16 x 64K 650 ->
   // 639, one of 32K 30.2 / 30.4 (with a ring of 3: 58.1, 39.5, 640 and 30.8); so does the

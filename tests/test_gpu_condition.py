@@ -9,8 +9,8 @@ condition lies within 1e-3 relative (plus 1e-5 absolute) of eps; outputs within
 GPU's own selection; statistics and routing counts exact.
 
 The decode tests run both implementations of the fused and fixed-mask entry points:
-the one-launch calls (``ia_condition_decode_fused``, ``ia_fixed_mask_decode_fused``,
-the default where a call fits one launch) and the multi-launch paths (statistics,
+the one-launch call (``ia_condition_one_launch``, with and without a mask, the default
+where a call fits one launch) and the multi-launch paths (statistics,
 route, finalize, merge; route, finalize, merge).
 """
 

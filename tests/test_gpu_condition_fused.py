@@ -1,8 +1,10 @@
-"""The one-launch condition call (``ia_condition_decode_fused``) beyond the parity
-cases that ``tests/test_gpu_condition.py`` runs on both implementations:
+"""The one-launch condition call for GQA groups of up to 4 (``ia_condition_one_launch``, and
+``ia_condition_decode_fused`` through the C ABI; groups of 8 are in
+``tests/test_gpu_condition_group8.py``) beyond the parity cases that
+``tests/test_gpu_condition.py`` runs on both implementations:
 
-* which calls fit one launch (GQA groups up to 4, rows x items within the device's
-  resident workgroups);
+* which calls ``ia_condition_decode_fused`` takes (groups of up to 4, rows x items within
+  the device's resident workgroups);
 * the statistics hand-off: with a wait limit of 0 every item computes the other
   items' partials itself, and selection and output equal the default run bit for
   bit (the result never depends on which workgroups run together);
@@ -48,7 +50,7 @@ def test_one_launch_eligibility(device):
     n = _items(1, 8, 4, 128, 2048, 64)
     assert 4 <= n <= 64, n                          # the reference's 128K configuration
     assert _items(1, 8, 4, 128, 512, 64) >= 1     # 32K
-    assert _items(1, 8, 8, 128, 512, 64) == 0     # G = 8 takes the four-launch path
+    assert _items(1, 8, 8, 128, 512, 64) == 0     # refused by this entry point
     assert _items(1, 8, 4, 96, 512, 64) == 0      # head_dim
     assert _items(64, 8, 4, 128, 2048, 64) == 0   # 512 rows x 4 items of 512 blocks: not resident at once
     assert _items(1, 2, 4, 128, 3, 64) <= 3       # never more items than blocks
