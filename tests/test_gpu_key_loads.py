@@ -61,10 +61,15 @@ def test_line_counts_the_blocks_a_row_can_choose(k, k_cap, in_k, whole, device):
     kw = dict(block_size=64, forced_first=1, forced_last=1, forced_in_k=in_k, k_cap=k_cap, score="quest", workspace={})
     ia.sparse_topk_decode(q, *pool, keys["quest"], k, **kw)
     torch.cuda.synchronize()
-    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU,
-                                            torch.profiler.ProfilerActivity.CUDA]) as prof:
-        ia.sparse_topk_decode(q, *pool, keys["quest"], k, **kw)
-        torch.cuda.synchronize()
+    prof = torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU,
+                                              torch.profiler.ProfilerActivity.CUDA])
+    try:
+        prof.start()
+    except RuntimeError as e:
+        pytest.skip(f"no profiler here: {e}")
+    ia.sparse_topk_decode(q, *pool, keys["quest"], k, **kw)
+    torch.cuda.synchronize()
+    prof.stop()
     names = [e.key for e in prof.key_averages() if "paged_finalize" in e.key]
     if not names:
         pytest.skip("the profiler recorded no kernels")

@@ -159,14 +159,16 @@ def test_line_between_one_launch_and_two(b, hkv, nb_max, device):
     n = b * hkv
     two = nb_max > 8192 or (1024 < nb_max <= 4096 if n >= 2 * cus else nb_max > max(1024, 8192 * n // cus))
     assert bool((rows[0, 0] != -1).any()) == two
+    full = ia.select_blocks_topk(q, kb, seq, 30, block_size=block, forced_first=2, forced_last=1, return_scores=True)
+    assert _same(full, got)
+    live = torch.arange(nb_max, device=device)[None, None] < nbs[:, None, None]
+    assert torch.equal(torch.isfinite(full[2]), live.expand_as(full[2])) and bool((full[2][~live.expand_as(full[2])] < 0).all())
     if nb_max <= 8192:
         assert _same(_one_launch(q, kb, seq, 30, block, 2, 1), got)
     else:
-        ref = ia.select_blocks_topk(q, kb, seq, 30, block_size=block, forced_first=2, forced_last=1,
-                                    return_scores=True)
         for i in (0, 5, b - 1):
             m = int(nbs[i])
-            sel = S.select_topk(ref[2][i, 0].cpu().numpy(), m, 30, 2, 1, False)
+            sel = S.select_topk(full[2][i, 0].cpu().numpy(), m, 30, 2, 1, False)
             assert np.array_equal(got[0][i, 0, :int(got[1][i, 0])].cpu().numpy(), sel)
 
 
